@@ -6,8 +6,10 @@
  * hipStream_t passed as void* (NULL = the default stream).  Every call is
  * stream-ordered and asynchronous unless its comment says it waits.  Every call returns NVQ_OK (0)
  * or a negative NVQ_ERR_* status.  Nothing throws across the ABI.  Query scratch (ray-tile orders,
- * queue counters, the sort buffers of binned point queries) lives in one grow-only block per
- * (device, stream) that the library keeps until the process ends; besides it, the library holds
+ * queue counters, slot maps of ray queries: about 3 KB per leaf, the sort buffers of binned point
+ * queries) lives in one grow-only block per (device, stream) that the library keeps until the
+ * process ends; ray queries take no slot map on a stream under graph capture, or where the block
+ * cannot grow, and give the same bits without it.  Besides the block, the library holds
  * the opt-in kernel profiler (nvq_profile_*), the work-queue array of nvq_multi_query_noalloc and
  * a small pinned host buffer per calling thread for values it reads back.  Calls on distinct
  * streams are thread-safe; calls on one stream from several threads are serialised.  The caller

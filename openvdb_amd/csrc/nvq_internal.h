@@ -311,13 +311,17 @@ private:
 
 // The longest-first order of a ray launch (nullptr up to kOrderMinTiles tiles), in the stream's
 // workspace, with `extra` more bytes, 256-byte aligned, for the caller.
+struct SlotMap;
 struct TileOrder {
     WorkspaceLease lease;
     const uint32_t* order = nullptr;
     char* extra = nullptr;
+    bool map = false; // a slot map of the grid was built
 };
+// With `map`, also the grid's slot map (nvq_slots.h), where the rule on its size, the scratch and the
+// stream allow it: a stream under graph capture takes none.
 int tileOrder(const GridView& g, const float* eye, const float* dir, const Sched& s, TileOrder& out, hipStream_t st,
-              size_t extraBytes = 0);
+              size_t extraBytes = 0, SlotMap* map = nullptr);
 
 
 // Large-batch point sampling through spatial bins and LDS bricks (nvq_binned.hip).

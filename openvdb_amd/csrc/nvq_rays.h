@@ -1,6 +1,7 @@
 // Per-ray query bodies shared by the single-grid kernels and the persistent multi-grid kernel.
 #pragma once
 #include "nvq_device.h"
+#include "nvq_slots.h"
 
 namespace nvq {
 
@@ -79,6 +80,95 @@ __device__ __forceinline__ void fogMarchRay(const GridView& g, const float* __re
     });
     if (Lout) Lout[i] = L;
     if (Tout) Tout[i] = T;
+}
+
+// The same march over a slot map (marchSteps step for step: same cells, positions and operations, so
+// the same bits).  Steps of a slot are taken kMarchBatch at a time: their positions do not depend
+// on the samples, so all their loads are in flight before the first is composited.  Returns false,
+// with nothing written, when the ray meets a slot the map does not resolve.
+//
+// Bound by the L1's line rate and the VALU in turn: per step four 8-byte loads that touch the
+// lines of 64 neighbouring cells, and about 60 instructions.  A batch of 4 hides the loads' latency
+// where few wavefronts are resident (57,600 rays: 0.24 ms at 2, 0.20 ms at 4) and costs nothing in a
+// full launch (1024^2 rays: 1.34 ms at 2, 1.29 ms at 4).
+constexpr int kMarchBatch = 4;
+
+template<int B>
+__device__ __forceinline__ bool fogMarchSlots(const SlotMap& M, const GridView& g, const float* __restrict__ eye,
+                                              const float* __restrict__ dir, uint64_t i, float dt, float sigma,
+                                              float* __restrict__ Lout, float* __restrict__ Tout)
+{
+    const float e[3] = {eye[3 * i], eye[3 * i + 1], eye[3 * i + 2]};
+    const float d[3] = {dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]};
+    float L = 0.0f, T = 1.0f;
+    Ray R = worldToIndexRay(g, e, d);
+    const float Eps = 0.000001f, Delta = 0.01f;
+    bool in = rayClip(R, g.bbox) && !(double(R.t1) > 1e20);
+    const float t0 = R.t0 + Eps, t1 = R.t1 - Eps;
+    in = in && !(t0 > t1);
+    if (in) {
+        float p[3];
+        rayAt(R, t0, p);
+        SlotCell c;
+        if (!slotCell(M, ifloor(p[0]), ifloor(p[1]), ifloor(p[2]), c)) return false;
+        HDDA h;
+        h.init(R, t0, t1, c.dim > 8 ? c.dim : 8);
+        for (;;) {
+            const float ta = h.t0;
+            const bool more = h.stepOnce();
+            const float tb = fminf(h.t0, t1);
+            const bool brick = !(c.entry & kSlotTile);
+            if ((brick || (c.entry & kSlotTileOn)) && ta < tb) {
+                const uint32_t base = brick ? c.entry * kBrickFloats : 0u;
+                float kf = ceilf(ta / dt);
+                float t = kf * dt;
+                while (t < tb) {
+                    float x[B][3];
+                    bool ok[B], fast[B];
+                    Cell cell[B];
+                    ok[0] = true;
+#pragma unroll
+                    for (int j = 0; j < B; ++j) {
+                        if (j) {
+                            const float kn = kf + 1.0f;
+                            t = kn * dt;
+                            ok[j] = ok[j - 1] && kn != kf && t < tb; // kn == kf: beyond 2^24 steps
+                            kf = kn;
+                        }
+                        x[j][0] = __builtin_fmaf(t, R.dir[0], R.eye[0]);
+                        x[j][1] = __builtin_fmaf(t, R.dir[1], R.eye[1]);
+                        x[j][2] = __builtin_fmaf(t, R.dir[2], R.eye[2]);
+                        const uint32_t rx = uint32_t(ifloor(x[j][0]) - c.ox), ry = uint32_t(ifloor(x[j][1]) - c.oy),
+                                       rz = uint32_t(ifloor(x[j][2]) - c.oz);
+                        fast[j] = brick && (rx | ry | rz) < 8u;
+                        brickCell(M, fast[j] ? base + (rx * 9u + ry) * 9u + rz : 0u, cell[j]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < B; ++j) {
+                        if (!ok[j]) continue;
+                        const float fx = floorf(x[j][0]), fy = floorf(x[j][1]), fz = floorf(x[j][2]);
+                        float rho = trilerp(cell[j], x[j][0] - fx, x[j][1] - fy, x[j][2] - fz);
+                        // a tile, or a position that rounding put just outside its slot
+                        if (!fast[j] && !slotTrilinear(M, x[j][0], x[j][1], x[j][2], rho)) return false;
+                        const float a = stepAbsorption(sigma, rho, dt);
+                        L += T * (1.0f - a) * rho;
+                        T *= a;
+                    }
+                    const float kn = kf + 1.0f;
+                    if (!ok[B - 1] || kn == kf) break;
+                    kf = kn;
+                    t = kf * dt;
+                }
+            }
+            if (!more) break;
+            rayAt(R, h.t0 + Delta, p);
+            if (!slotCell(M, ifloor(p[0]), ifloor(p[1]), ifloor(p[2]), c)) return false;
+            h.update(R, c.dim > 8 ? c.dim : 8);
+        }
+    }
+    if (Lout) Lout[i] = L;
+    if (Tout) Tout[i] = T;
+    return true;
 }
 
 } // namespace nvq

@@ -1,0 +1,226 @@
+// Slot maps (nvq_slots.h): the flattened view of a grid that the ray queries read.
+//   k_slot_entries : one tree walk per 8^3 slot of the bbox
+//   k_slot_bricks  : one wavefront per leaf decodes its 9^3 brick
+#include "nvq_slots.h"
+#include "nvq_internal.h"
+#include "nvq_profile.h"
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+namespace nvq {
+namespace {
+
+constexpr int kThreads = 256;
+
+template<uint32_t GT>
+__global__ __launch_bounds__(kThreads) void k_slot_entries(GridView g, SlotMap M, uint32_t count,
+                                                           uint32_t* __restrict__ entry, float* __restrict__ value,
+                                                           uint32_t* __restrict__ slotOf,
+                                                           uint32_t* __restrict__ leafOff,
+                                                           uint32_t* __restrict__ leaves)
+{
+    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+    if (i >= count) return;
+    const uint32_t z = i % M.n[2], r = i / M.n[2], y = r % M.n[1], x = r / M.n[1];
+    Accessor<GT> acc(g);
+    const Probe p = acc.probe((M.lo[0] + int32_t(x)) << 3, (M.lo[1] + int32_t(y)) << 3, (M.lo[2] + int32_t(z)) << 3);
+    uint32_t e;
+    if (!p.leaf) {
+        e = kSlotTile | (p.active ? kSlotTileOn : 0u) | (p.dim == 8u ? 0u : (p.dim == 128u ? 1u : 2u));
+    } else if (p.dim != 1u || x + 1u >= M.n[0] || y + 1u >= M.n[1] || z + 1u >= M.n[2]) {
+        e = kSlotOther;
+    } else {
+        // bricks are numbered as the leaves are, where these have one size; FpN's are numbered as
+        // the threads come (any order gives the same outputs).  A leaf outside the leaf array
+        // (not laid out breadth first) has no number.
+        const uint64_t off = uint64_t(p.leaf - g.leaf0);
+        if constexpr (GT == GT_FPN) {
+            e = kSlotOther;
+            if ((off & 31u) == 0 && off < (uint64_t(1) << 37)) {
+                const uint32_t b = atomicAdd(leaves, 1u);
+                if (b < g.leafCount) {
+                    leafOff[b] = uint32_t(off >> 5);
+                    e = b;
+                }
+            }
+        } else {
+            const uint64_t b = off / g.leafSize;
+            e = b < g.leafCount && b * g.leafSize == off ? uint32_t(b) : kSlotOther;
+        }
+    }
+    entry[i] = e;
+    value[i] = p.value;
+    if (!(e & kSlotTile)) slotOf[e] = i;
+}
+
+// Decoded values of the eight voxels (x, y, 0..7) of a leaf, row = 8 x + y: one or two wide loads.
+template<uint32_t GT>
+__device__ __forceinline__ void leafRow(const uint8_t* leaf, uint32_t row, const float* channel, float v[8])
+{
+    if constexpr (GT == GT_FLOAT) {
+        const float4* p = reinterpret_cast<const float4*>(leaf + kLeafData + 32u * row);
+        const float4 a = p[0], b = p[1];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else if constexpr (GT == GT_FP16 || GT == GT_FP8 || GT == GT_FP4) {
+        constexpr int kBits = GT == GT_FP16 ? 16 : (GT == GT_FP8 ? 8 : 4), kWords = kBits / 4;
+        uint32_t w[kWords];
+        __builtin_memcpy(w, leaf + kLeafData + row * uint32_t(kBits), sizeof(w));
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            v[k] = dequant(leaf, (w[k * kBits / 32] >> (k * kBits % 32)) & ((1u << kBits) - 1u));
+    } else if constexpr (GT == GT_ONINDEX) {
+        // the row is one byte of the value mask: its active voxels have consecutive indices
+        const uint32_t w = row >> 3, shift = 8u * (row & 7u);
+        const uint64_t word = ld_u64(leaf + kLeafVMask + 8u * w);
+        uint64_t at = ld_u64(leaf + kIdxLeafOffset) + uint64_t(__popcll(word & ((uint64_t(1) << shift) - 1u)));
+        if (w) at += (ld_u64(leaf + kIdxLeafPrefix) >> (9u * (w - 1u))) & 511u;
+        const uint32_t bits = uint32_t(word >> shift) & 255u;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const bool on = (bits >> k) & 1u;
+            v[k] = channel[on ? at : 0u];
+            at += on ? 1u : 0u;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = Codec<GT>::get(leaf, 8u * row + k, channel);
+    }
+}
+
+// One wavefront per brick.  Lane l decodes row (x, y) = (l / 8, l % 8) of the leaf, one voxel of
+// each facing layer of the three upper neighbours and, lanes 0..24, one of the layers' edges and
+// corner; the brick is put together in LDS and written as whole 16-byte words.  All loads of a
+// lane are independent.  Bound by HBM: the leaves are read and the bricks written once.
+// One wavefront for the leaves of 16 slots in turn, each voxel on its own: 548 us for the
+// 141,950 leaves of a 512^3 fog.
+template<uint32_t GT>
+__global__ __launch_bounds__(kThreads) void k_slot_bricks(GridView g, SlotMap M, uint32_t count,
+                                                          const uint32_t* __restrict__ slotOf,
+                                                          const uint32_t* __restrict__ leafOff,
+                                                          float* __restrict__ brick)
+{
+    __shared__ __align__(16) float stage[kThreads / 64][kBrickFloats];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t b = __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + wv);
+    if (b >= g.leafCount) return; // whole wavefronts; no barrier follows
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(slotOf[b]);
+    // a number no slot was given (its leaf lies outside the table) holds what was there before
+    if (slot >= count || M.entry[slot] != b) return;
+    float* out = stage[wv];
+    auto leafOf = [&](uint32_t e) {
+        return g.leaf0 + (GT == GT_FPN ? uint64_t(leafOff[e]) << 5 : uint64_t(e) * g.leafSize);
+    };
+    // voxel (x, y, z) of the brick that lies in the neighbour slot above on the axes given
+    auto beyond = [&](uint32_t x, uint32_t y, uint32_t z) -> float {
+        // leaves on the table's rim are kSlotOther: the slot above exists on every axis
+        const uint32_t s = slot + ((x >> 3) * M.n[1] + (y >> 3)) * M.n[2] + (z >> 3);
+        const uint32_t e = M.entry[s];
+        if (!(e & kSlotTile)) return Codec<GT>::get(leafOf(e), ((x & 7u) << 6) | ((y & 7u) << 3) | (z & 7u), g.channel);
+        if (e != kSlotOther) return M.value[s];
+        // a neighbour the table does not resolve: through the tree
+        Accessor<GT> acc(g);
+        const uint32_t sz = slot % M.n[2], r = slot / M.n[2], sy = r % M.n[1], sx = r / M.n[1];
+        return acc.getValue(((M.lo[0] + int32_t(sx)) << 3) + int32_t(x), ((M.lo[1] + int32_t(sy)) << 3) + int32_t(y),
+                            ((M.lo[2] + int32_t(sz)) << 3) + int32_t(z));
+    };
+    const uint32_t h = lane >> 3, l = lane & 7u;
+    float row[8];
+    leafRow<GT>(leafOf(b), lane, g.channel, row);
+    const float fx = beyond(8u, h, l), fy = beyond(h, 8u, l), fz = beyond(h, l, 8u);
+    // lanes 0..7: (8, l, 8); 8..15: (l, 8, 8); 16..23: (8, 8, l); 24: (8, 8, 8)
+    const uint32_t ex = h == 1 ? l : 8u, ey = h == 0 ? l : 8u, ez = h == 2 ? l : 8u;
+    const float fe = lane < 25u ? beyond(ex, ey, ez) : 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) out[h * 81u + l * 9u + k] = row[k];
+    out[8u * 81u + h * 9u + l] = fx;
+    out[h * 81u + 8u * 9u + l] = fy;
+    out[h * 81u + l * 9u + 8u] = fz;
+    if (lane < 25u) out[ex * 81u + ey * 9u + ez] = fe;
+    __builtin_amdgcn_wave_barrier(); // the wavefront reads what its own lanes wrote, in LDS order
+    const float4* src = reinterpret_cast<const float4*>(out);
+    float4* dst = reinterpret_cast<float4*>(brick + uint64_t(b) * kBrickFloats);
+#pragma unroll
+    for (uint32_t j = 0; j < 3; ++j) {
+        const uint32_t k = j * 64u + lane;
+        if (k < (kBrickEdge * kBrickEdge * kBrickEdge + 3u) / 4u) dst[k] = src[k];
+    }
+}
+
+__global__ void k_zero_word(uint32_t* p) { *p = 0u; }
+
+bool slotBox(const GridView& g, int32_t lo[3], uint32_t n[3], uint64_t& count)
+{
+    count = 1;
+    for (int a = 0; a < 3; ++a) {
+        // empty grids, and coordinates whose neighbours could leave the int32 range
+        if (g.bbox[a] > g.bbox[3 + a] || g.bbox[a] < -(1 << 30) || g.bbox[3 + a] > (1 << 30)) return false;
+        const int64_t l = (int64_t(g.bbox[a]) >> 3) - 1, h = (int64_t(g.bbox[3 + a]) >> 3) + 2;
+        lo[a] = int32_t(l);
+        n[a] = uint32_t(h - l + 1);
+        count *= n[a];
+        if (count > kMaxMapSlots) return false;
+    }
+    return true;
+}
+
+size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
+
+template<uint32_t GT>
+void launchMap(const GridView& g, const SlotMap& M, uint32_t count, uint32_t* entry, float* value, float* brick,
+               uint32_t* slotOf, uint32_t* leafOff, uint32_t* leaves, hipStream_t s)
+{
+    if (GT == GT_FPN) hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, leaves);
+    hipLaunchKernelGGL(k_slot_entries<GT>, dim3((count + kThreads - 1) / kThreads), dim3(kThreads), 0, s, g, M, count,
+                       entry, value, slotOf, leafOff, leaves);
+    if (g.leafCount)
+        hipLaunchKernelGGL(k_slot_bricks<GT>, dim3((g.leafCount + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0,
+                           s, g, M, count, slotOf, leafOff, brick);
+}
+
+} // namespace
+
+size_t slotMapBytes(const GridView& g, uint64_t rays)
+{
+    int32_t lo[3];
+    uint32_t n[3];
+    uint64_t count;
+    if (!slotBox(g, lo, n, count)) return 0;
+    if (count > kMapSlotsPerRay * rays + kMapSlotsFree || g.leafCount > kMapLeavesPerRay * rays + kMapLeavesFree ||
+        g.leafCount > kMaxMapLeaves)
+        return 0;
+    const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
+    return up256(4 * count) * 2 + up256(4 * leaves) * 2 + 256 + up256(4ull * kBrickFloats * leaves);
+}
+
+int launchSlotMap(const GridView& g, char* mem, SlotMap& M, hipStream_t s)
+{
+    uint64_t count;
+    if (!slotBox(g, M.lo, M.n, count)) return -1;
+    const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
+    uint32_t* entry = reinterpret_cast<uint32_t*>(mem);
+    float* value = reinterpret_cast<float*>(mem + up256(4 * count));
+    uint32_t* slotOf = reinterpret_cast<uint32_t*>(mem + 2 * up256(4 * count));
+    uint32_t* leafOff = reinterpret_cast<uint32_t*>(mem + 2 * up256(4 * count) + up256(4 * leaves));
+    uint32_t* number = reinterpret_cast<uint32_t*>(mem + 2 * up256(4 * count) + 2 * up256(4 * leaves));
+    float* brick = reinterpret_cast<float*>(number + 64);
+    M.entry = entry;
+    M.value = value;
+    M.brick = brick;
+    ProfScope prof("slot_map", s);
+    const uint32_t c = uint32_t(count);
+    switch (g.type) {
+    case GT_FLOAT: launchMap<GT_FLOAT>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    case GT_FP4: launchMap<GT_FP4>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    case GT_FP8: launchMap<GT_FP8>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    case GT_FP16: launchMap<GT_FP16>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    case GT_FPN: launchMap<GT_FPN>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    case GT_ONINDEX: launchMap<GT_ONINDEX>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    default: return -3;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -4;
+}
+
+} // namespace nvq
