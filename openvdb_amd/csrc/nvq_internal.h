@@ -316,12 +316,13 @@ struct TileOrder {
     WorkspaceLease lease;
     const uint32_t* order = nullptr;
     char* extra = nullptr;
-    bool map = false; // a slot map of the grid was built
+    bool map = false;        // a slot map of the grid was built
+    char* withMap = nullptr; // the scratch asked for beside it, 256-byte aligned
 };
-// With `map`, also the grid's slot map (nvq_slots.h), where the rule on its size, the scratch and the
-// stream allow it: a stream under graph capture takes none.
+// With `map`, also the grid's slot map (nvq_slots.h) and `withMapBytes` of scratch, where the rule on
+// its size, the scratch and the stream allow it: a stream under graph capture takes none.
 int tileOrder(const GridView& g, const float* eye, const float* dir, const Sched& s, TileOrder& out, hipStream_t st,
-              size_t extraBytes = 0, SlotMap* map = nullptr);
+              size_t extraBytes = 0, SlotMap* map = nullptr, size_t withMapBytes = 0);
 
 
 // Large-batch point sampling through spatial bins and LDS bricks (nvq_binned.hip).

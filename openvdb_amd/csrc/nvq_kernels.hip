@@ -483,7 +483,7 @@ char* nvq::WorkspaceLease::acquire(size_t bytes, hipStream_t s)
 }
 
 int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const Sched& s, TileOrder& out, hipStream_t st,
-                   size_t extraBytes, SlotMap* map)
+                   size_t extraBytes, SlotMap* map, size_t withMapBytes)
 {
     if (s.tiles == 0 || s.tiles > (uint64_t(1) << 32)) return -1;
     const bool ordered = s.tiles > kOrderMinTiles;
@@ -496,14 +496,16 @@ int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const 
     // a captured launch must not depend on scratch that a later call on the stream may replace
     if (mapBytes && (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone))
         mapBytes = 0;
+    mapBytes = (mapBytes + 255) & ~size_t(255);
     char* base = nullptr;
-    if (mapBytes && !(base = out.lease.acquire(mapAt + mapBytes, st))) mapBytes = 0;
+    if (mapBytes && !(base = out.lease.acquire(mapAt + mapBytes + withMapBytes, st))) mapBytes = 0;
     if (!base && mapAt) {
         base = out.lease.acquire(mapAt, st);
         if (!base) return -1;
     }
     out.extra = extraBytes ? base + keyBytes + orderBytes + countBytes : nullptr;
     out.map = mapBytes != 0;
+    out.withMap = mapBytes && withMapBytes ? base + mapAt + mapBytes : nullptr;
     if (mapBytes && launchSlotMap(g, base + mapAt, *map, st) != 0) return -1;
     if (!ordered) {
         out.order = nullptr;

@@ -31,6 +31,7 @@ struct SlotMap {
     const uint32_t* entry;
     const float* value;
     const float* brick;
+    const uint32_t* tileIndex; // index grids: the channel index of a slot without a leaf
 };
 
 // One slot as a march or crossing meets it.

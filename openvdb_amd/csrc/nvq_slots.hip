@@ -17,6 +17,7 @@ constexpr int kThreads = 256;
 template<uint32_t GT>
 __global__ __launch_bounds__(kThreads) void k_slot_entries(GridView g, SlotMap M, uint32_t count,
                                                            uint32_t* __restrict__ entry, float* __restrict__ value,
+                                                           uint32_t* __restrict__ tileIndex,
                                                            uint32_t* __restrict__ slotOf,
                                                            uint32_t* __restrict__ leafOff,
                                                            uint32_t* __restrict__ leaves)
@@ -53,6 +54,7 @@ __global__ __launch_bounds__(kThreads) void k_slot_entries(GridView g, SlotMap M
     entry[i] = e;
     value[i] = p.value;
     if (!(e & kSlotTile)) slotOf[e] = i;
+    if constexpr (GT == GT_ONINDEX) tileIndex[i] = uint32_t(p.index); // used by the adjoint: < 2^31 values
 }
 
 // Decoded values of the eight voxels (x, y, 0..7) of a leaf, row = 8 x + y: one or two wide loads.
@@ -169,12 +171,12 @@ bool slotBox(const GridView& g, int32_t lo[3], uint32_t n[3], uint64_t& count)
 size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
 template<uint32_t GT>
-void launchMap(const GridView& g, const SlotMap& M, uint32_t count, uint32_t* entry, float* value, float* brick,
-               uint32_t* slotOf, uint32_t* leafOff, uint32_t* leaves, hipStream_t s)
+void launchMap(const GridView& g, const SlotMap& M, uint32_t count, uint32_t* entry, float* value, uint32_t* tileIndex,
+               float* brick, uint32_t* slotOf, uint32_t* leafOff, uint32_t* leaves, hipStream_t s)
 {
     if (GT == GT_FPN) hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, leaves);
     hipLaunchKernelGGL(k_slot_entries<GT>, dim3((count + kThreads - 1) / kThreads), dim3(kThreads), 0, s, g, M, count,
-                       entry, value, slotOf, leafOff, leaves);
+                       entry, value, tileIndex, slotOf, leafOff, leaves);
     if (g.leafCount)
         hipLaunchKernelGGL(k_slot_bricks<GT>, dim3((g.leafCount + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0,
                            s, g, M, count, slotOf, leafOff, brick);
@@ -192,7 +194,8 @@ size_t slotMapBytes(const GridView& g, uint64_t rays)
         g.leafCount > kMaxMapLeaves)
         return 0;
     const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
-    return up256(4 * count) * 2 + up256(4 * leaves) * 2 + 256 + up256(4ull * kBrickFloats * leaves);
+    return up256(4 * count) * (g.type == GT_ONINDEX ? 3 : 2) + up256(4 * leaves) * 2 + 256 +
+           up256(4ull * kBrickFloats * leaves);
 }
 
 int launchSlotMap(const GridView& g, char* mem, SlotMap& M, hipStream_t s)
@@ -200,24 +203,32 @@ int launchSlotMap(const GridView& g, char* mem, SlotMap& M, hipStream_t s)
     uint64_t count;
     if (!slotBox(g, M.lo, M.n, count)) return -1;
     const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
-    uint32_t* entry = reinterpret_cast<uint32_t*>(mem);
-    float* value = reinterpret_cast<float*>(mem + up256(4 * count));
-    uint32_t* slotOf = reinterpret_cast<uint32_t*>(mem + 2 * up256(4 * count));
-    uint32_t* leafOff = reinterpret_cast<uint32_t*>(mem + 2 * up256(4 * count) + up256(4 * leaves));
-    uint32_t* number = reinterpret_cast<uint32_t*>(mem + 2 * up256(4 * count) + 2 * up256(4 * leaves));
-    float* brick = reinterpret_cast<float*>(number + 64);
+    char* at = mem;
+    auto take = [&](size_t bytes) {
+        char* p = at;
+        at += up256(bytes);
+        return p;
+    };
+    uint32_t* entry = reinterpret_cast<uint32_t*>(take(4 * count));
+    float* value = reinterpret_cast<float*>(take(4 * count));
+    uint32_t* index = g.type == GT_ONINDEX ? reinterpret_cast<uint32_t*>(take(4 * count)) : nullptr;
+    uint32_t* slotOf = reinterpret_cast<uint32_t*>(take(4 * leaves));
+    uint32_t* leafOff = reinterpret_cast<uint32_t*>(take(4 * leaves));
+    uint32_t* number = reinterpret_cast<uint32_t*>(take(4));
+    float* brick = reinterpret_cast<float*>(take(4ull * kBrickFloats * leaves));
     M.entry = entry;
     M.value = value;
     M.brick = brick;
+    M.tileIndex = index;
     ProfScope prof("slot_map", s);
     const uint32_t c = uint32_t(count);
     switch (g.type) {
-    case GT_FLOAT: launchMap<GT_FLOAT>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
-    case GT_FP4: launchMap<GT_FP4>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
-    case GT_FP8: launchMap<GT_FP8>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
-    case GT_FP16: launchMap<GT_FP16>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
-    case GT_FPN: launchMap<GT_FPN>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
-    case GT_ONINDEX: launchMap<GT_ONINDEX>(g, M, c, entry, value, brick, slotOf, leafOff, number, s); break;
+    case GT_FLOAT: launchMap<GT_FLOAT>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
+    case GT_FP4: launchMap<GT_FP4>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
+    case GT_FP8: launchMap<GT_FP8>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
+    case GT_FP16: launchMap<GT_FP16>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
+    case GT_FPN: launchMap<GT_FPN>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
+    case GT_ONINDEX: launchMap<GT_ONINDEX>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
     default: return -3;
     }
     return hipGetLastError() == hipSuccess ? 0 : -4;

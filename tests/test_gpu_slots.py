@@ -1,4 +1,5 @@
-"""The fog march over a slot map against the same march through the accessor, bit for bit.
+"""The fog march over a slot map against the same march through the accessor, bit for bit, and its
+adjoint (2x2x2 blocks in LDS) against the FP64 oracle and across schedules and grid types.
 
 A launch under graph capture takes no scratch and goes through the accessor, so a captured call is
 the reference here; the march itself is compared with the FP64 oracle in test_gpu_parity.py.
@@ -86,3 +87,61 @@ def test_march_over_slots_equals_march_through_the_accessor(name, codec):
             assert torch.equal(L, L2)
         if n > 64:
             assert float(L.max()) > 0.0
+
+
+@pytest.fixture(scope="module")
+def oracle():
+    from pyoracle import Oracle
+    return Oracle()
+
+
+def _image(d, w, h):
+    lo, hi = np.array(d.index_bbox[:3], np.float64), np.array(d.index_bbox[3:], np.float64) + 1
+    eye = 0.5 * (lo + hi) + 1.1 * np.linalg.norm(hi - lo) * np.array([0.48, -0.36, 0.8])
+    e, r = _nvq().tools.camera_rays(w, h, tuple(eye), tuple(0.5 * (lo + hi)), (0.0, 1.0, 0.0), 45.0)
+    return torch.from_numpy(e).cuda(), torch.from_numpy(r).cuda()
+
+
+@pytest.mark.parametrize("name,w,h", [("fog", 1, 1), ("fog", 40, 27), ("fog", 203, 161), ("tiles", 61, 50),
+                                      ("fog_sphere", 61, 50), ("flagged", 61, 50)])
+def test_adjoint_over_blocks(oracle, name, w, h):
+    nvq = _nvq()
+    host = _host(nvq, name)
+    d = nvq.DeviceGrid(host)
+    eye, dirs = _image(d, w, h)
+    r = torch.Generator(device="cuda")
+    r.manual_seed(w)
+    gL, gT = (torch.randn(w * h, generator=r, device="cuda") for _ in range(2))
+    gL[::7] = 0.0
+    gT[::7] = 0.0  # rays without a gradient idle beside the others
+    L, T = nvq.ops.fog_march(d, eye, dirs, 0.5, 0.05, image_width=w)
+    acc = nvq.ops.fog_march_backward(d, eye, dirs, L, gL, T, gT, 0.5, 0.05, image_width=w)
+    # integer sums: other wavefronts, other blocks in each cache, the same result
+    order = torch.randperm(w * h, generator=r, device="cuda")
+    mixed = [x[order].contiguous() for x in (eye, dirs, L, gL, T, gT)]
+    assert torch.equal(acc, nvq.ops.fog_march_backward(d, *mixed, 0.5, 0.05))
+    g = nvq.ops.fixed_to_float(acc).double().cpu().numpy()
+    want = oracle.fog_march_adjoint(host, eye.cpu().numpy(), dirs.cpu().numpy(), 0.5, 0.05,
+                                    gL.double().cpu().numpy(), gT.double().cpu().numpy())
+    assert np.abs(g - want).max() <= 1e-4 * np.abs(want).max()  # the bound of the accessor adjoint's test
+    if name == "fog":
+        # the same voxels as an index grid: entry by entry the same integers
+        ijk, values = nvq.tools.active_voxels(host)
+        i, index = nvq.DeviceGrid.from_voxels(torch.from_numpy(ijk).cuda(), "OnIndex", return_index=True)
+        channel = torch.zeros(i.value_count, device="cuda")
+        channel[index] = torch.from_numpy(values).cuda()
+        i.set_channel(channel)
+        Li, Ti = nvq.ops.fog_march(i, eye, dirs, 0.5, 0.05, image_width=w)
+        assert torch.equal(L, Li) and torch.equal(T, Ti)
+        acci = nvq.ops.fog_march_backward(i, eye, dirs, L, gL, T, gT, 0.5, 0.05, image_width=w)
+        mask = np.unpackbits(host[_leaf_bytes(host)].reshape(-1, 2144)[:, 16:80], axis=1, bitorder="little")
+        on = torch.from_numpy(np.flatnonzero(mask.reshape(-1))).cuda()
+        assert torch.equal(acc[on], acci[index])
+        off = torch.from_numpy(np.flatnonzero(mask.reshape(-1) == 0)).cuda()
+        if w > 1:
+            assert int(acc[off].ne(0).sum()) > 0 and int(acci[0]) != 0  # the inactive voxels' sums
+
+
+def _leaf_bytes(host):
+    off, count = 672 + int(np.frombuffer(host, np.int64, 1, 672)[0]), int(np.frombuffer(host, np.uint32, 1, 704)[0])
+    return slice(off, off + 2144 * count)
