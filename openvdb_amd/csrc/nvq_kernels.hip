@@ -173,13 +173,24 @@ __global__ __launch_bounds__(kBlock) void k_grad_stencil(GridView g, const int32
 template<uint32_t GT>
 __global__ __launch_bounds__(kBlock) void k_zero_crossing(GridView g, const float* __restrict__ eye,
                                                           const float* __restrict__ dir, Sched s, float iso,
-                                                          uint8_t* __restrict__ hit, int32_t* __restrict__ ijk,
-                                                          float* __restrict__ tout, float* __restrict__ vout,
-                                                          float* __restrict__ normal)
+                                                          CrossingOut o)
 {
     uint64_t i;
     if (!schedule(s, i)) return;
-    zeroCrossingRay<GT>(g, eye, dir, i, iso, hit, ijk, tout, vout, normal);
+    zeroCrossingRay<GT>(g, eye, dir, i, iso, o);
+}
+
+// Over a slot map.  Rays that the map leaves open start over through the accessor (`whole`: the view in
+// device memory, so that its fields are not kept in registers for it).
+template<uint32_t GT>
+__global__ __launch_bounds__(kBlock) void k_zero_crossing_slots(SlotMap M, GridView g, const GridView* whole,
+                                                                const float* __restrict__ eye,
+                                                                const float* __restrict__ dir, Sched s, float iso,
+                                                                CrossingOut o)
+{
+    uint64_t i;
+    if (!schedule(s, i)) return;
+    if (!zeroCrossingSlots(M, g, eye, dir, i, iso, o)) zeroCrossingRay<GT>(*whole, eye, dir, i, iso, o);
 }
 
 // 75 VGPRs uncapped (6 wavefronts per SIMD).  Capped at 8 wavefronts (64 VGPRs, a 28-byte spill):
@@ -201,7 +212,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 // 1.29 ms here and 0.16 ms for the map; 320x180 rays through a 128^3 index grid 2.50 -> 0.20 ms.
 // Caps of 5 and 6 wavefronts (2 steps in flight, spills) were slower: 1.34 and 1.45 ms.
 template<uint32_t GT>
-__global__ __launch_bounds__(kBlock) void k_fog_march_slots(SlotMap M, GridView g, const float* __restrict__ eye,
+__global__ __launch_bounds__(kBlock) void k_fog_march_slots(SlotMap M, GridView g, const GridView* whole, const float* __restrict__ eye,
                                                             const float* __restrict__ dir, Sched s,
                                                             const uint32_t* __restrict__ order, float dt, float sigma,
                                                             float* __restrict__ Lout, float* __restrict__ Tout)
@@ -209,7 +220,7 @@ __global__ __launch_bounds__(kBlock) void k_fog_march_slots(SlotMap M, GridView 
     uint64_t i;
     if (!scheduleOrdered(s, order, i)) return;
     if (!fogMarchSlots<kMarchBatch>(M, g, eye, dir, i, dt, sigma, Lout, Tout))
-        fogMarchRay<GT>(g, eye, dir, i, dt, sigma, Lout, Tout);
+        fogMarchRay<GT>(*whole, eye, dir, i, dt, sigma, Lout, Tout);
 }
 
 // ------------------------------------------------------------------ longest-first tile order
@@ -277,22 +288,26 @@ template<uint32_t GT> struct RunGradStencil {
     }
 };
 template<uint32_t GT> struct RunZeroCrossing {
-    static void run(const GridView& g, const float* eye, const float* dir, const Sched& sc, float iso, uint8_t* hit,
-                    int32_t* ijk, float* t, float* v, float* nrm, hipStream_t s)
+    static void run(const GridView& g, const GridView* dg, const SlotMap* M, const float* eye, const float* dir,
+                    const Sched& sc, float iso,
+                    const CrossingOut& o, hipStream_t s)
     {
         ProfScope prof("k_zero_crossing", s);
-        hipLaunchKernelGGL(k_zero_crossing<GT>, dim3(launchBlocks(sc)), dim3(kBlock), 0, s, g, eye, dir, sc, iso, hit,
-                           ijk, t, v, nrm);
+        if (M)
+            hipLaunchKernelGGL(k_zero_crossing_slots<GT>, dim3(launchBlocks(sc)), dim3(kBlock), 0, s, *M, g, dg, eye, dir,
+                               sc, iso, o);
+        else
+            hipLaunchKernelGGL(k_zero_crossing<GT>, dim3(launchBlocks(sc)), dim3(kBlock), 0, s, g, eye, dir, sc, iso, o);
     }
 };
 template<uint32_t GT> struct RunFogMarch {
-    static void run(const GridView& g, const SlotMap* M, const float* eye, const float* dir, const Sched& sc,
-                    const uint32_t* order, float dt, float sigma, float* L, float* T, hipStream_t s)
+    static void run(const GridView& g, const GridView* dg, const SlotMap* M, const float* eye, const float* dir,
+                    const Sched& sc, const uint32_t* order, float dt, float sigma, float* L, float* T, hipStream_t s)
     {
         ProfScope prof("k_fog_march", s);
         if (M)
-            hipLaunchKernelGGL(k_fog_march_slots<GT>, dim3(orderedBlocks(sc)), dim3(kBlock), 0, s, *M, g, eye, dir, sc,
-                               order, dt, sigma, L, T);
+            hipLaunchKernelGGL(k_fog_march_slots<GT>, dim3(orderedBlocks(sc)), dim3(kBlock), 0, s, *M, g, dg, eye, dir,
+                               sc, order, dt, sigma, L, T);
         else
             hipLaunchKernelGGL(k_fog_march<GT>, dim3(orderedBlocks(sc)), dim3(kBlock), 0, s, g, eye, dir, sc, order, dt,
                            sigma, L, T);
@@ -490,23 +505,18 @@ int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const 
     const size_t keyBytes = ordered ? (size_t(s.tiles) * 4 + 255) & ~size_t(255) : 0;
     const size_t orderBytes = keyBytes;
     const size_t countBytes = ordered ? orderScratchBytes(s.tiles) : 0;
-    const size_t mapAt = (keyBytes + orderBytes + countBytes + extraBytes + 255) & ~size_t(255);
-    size_t mapBytes = map ? slotMapBytes(g, s.n) : 0;
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    // a captured launch must not depend on scratch that a later call on the stream may replace
-    if (mapBytes && (hipStreamIsCapturing(st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone))
-        mapBytes = 0;
-    mapBytes = (mapBytes + 255) & ~size_t(255);
+    const size_t need = keyBytes + orderBytes + countBytes + extraBytes;
     char* base = nullptr;
-    if (mapBytes && !(base = out.lease.acquire(mapAt + mapBytes + withMapBytes, st))) mapBytes = 0;
-    if (!base && mapAt) {
-        base = out.lease.acquire(mapAt, st);
-        if (!base) return -1;
+    if (map) {
+        // what goes with the map lies before it
+        const size_t at = (need + 255) & ~size_t(255);
+        base = acquireWithMap(out.lease, g, s.n, kMapBricks, 0.0f, at + withMapBytes, *map, out.map, st);
+        out.withMap = out.map && withMapBytes ? base + at : nullptr;
+    } else if (need) {
+        base = out.lease.acquire(need, st);
     }
+    if (need && !base) return -1;
     out.extra = extraBytes ? base + keyBytes + orderBytes + countBytes : nullptr;
-    out.map = mapBytes != 0;
-    out.withMap = mapBytes && withMapBytes ? base + mapAt + mapBytes : nullptr;
-    if (mapBytes && launchSlotMap(g, base + mapAt, *map, st) != 0) return -1;
     if (!ordered) {
         out.order = nullptr;
         return 0;
@@ -520,6 +530,26 @@ int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const 
     }
     out.order = order;
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// Scratch of `need` bytes plus a slot map of `parts` for `rays` rays, where the rule on the map's size, the
+// scratch and the stream allow it (mapped; the base is then need bytes, 256-aligned, before it).
+char* nvq::acquireWithMap(WorkspaceLease& lease, const GridView& g, uint64_t rays, uint32_t parts, float iso, size_t need,
+                          SlotMap& M, bool& mapped, hipStream_t st)
+{
+    mapped = false;
+    need = (need + 255) & ~size_t(255);
+    const size_t mapBytes = slotMapBytes(g, rays, parts);
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    // a captured launch must not depend on scratch that a later call on the stream may replace
+    if (mapBytes && hipStreamIsCapturing(st, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
+        char* base = lease.acquire(need + mapBytes, st);
+        if (base) {
+            mapped = launchSlotMap(g, base + need, M, parts, iso, st) == 0;
+            return base;
+        }
+    }
+    return need ? lease.acquire(need, st) : nullptr;
 }
 
 // ======================================================================= C ABI
@@ -693,6 +723,17 @@ int nvq_grid_get_view(const nvq_grid* grid, void* host_view, uint64_t view_bytes
     return NVQ_OK;
 }
 
+static int crossing(const nvq_grid* grid, const float* eye, const float* dir, uint64_t n, uint32_t image_width, float iso,
+                    const CrossingOut& o, hipStream_t s)
+{
+    WorkspaceLease lease;
+    SlotMap M;
+    bool mapped = false;
+    (void)acquireWithMap(lease, grid->view, n, kMapSigns, iso, 0, M, mapped, s);
+    const Sched sc = makeSched(n, image_width);
+    return launchTyped<RunZeroCrossing>(grid->view.type, grid->view, grid->dview, mapped ? &M : nullptr, eye, dir, sc, iso, o, s);
+}
+
 int nvq_get_value(const nvq_grid* grid, const int32_t* ijk, uint64_t n, float* val, uint8_t* active, uint32_t* dim,
                   void* stream)
 {
@@ -733,9 +774,7 @@ int nvq_zero_crossing(const nvq_grid* grid, const float* eye, const float* dir, 
     if (image_width && n % image_width) return NVQ_ERR_INVALID_ARG;
     if (n == 0) return NVQ_OK;
     if (n > (uint64_t(1) << 38)) return NVQ_ERR_INVALID_ARG;
-    const Sched sc = makeSched(n, image_width);
-    return launchTyped<RunZeroCrossing>(grid->view.type, grid->view, eye, dir, sc, 0.0f, hit, ijk, t, v, normal,
-                                        S(stream));
+    return crossing(grid, eye, dir, n, image_width, 0.0f, CrossingOut{hit, ijk, t, v, normal}, S(stream));
 }
 
 int nvq_iso_crossing(const nvq_grid* grid, const float* eye, const float* dir, uint64_t n, uint32_t image_width,
@@ -745,9 +784,7 @@ int nvq_iso_crossing(const nvq_grid* grid, const float* eye, const float* dir, u
     if (image_width && n % image_width) return NVQ_ERR_INVALID_ARG;
     if (n == 0) return NVQ_OK;
     if (n > (uint64_t(1) << 38)) return NVQ_ERR_INVALID_ARG;
-    const Sched sc = makeSched(n, image_width);
-    return launchTyped<RunZeroCrossing>(grid->view.type, grid->view, eye, dir, sc, iso, hit, ijk, t, v, normal,
-                                        S(stream));
+    return crossing(grid, eye, dir, n, image_width, iso, CrossingOut{hit, ijk, t, v, normal}, S(stream));
 }
 
 int nvq_render_iso_surface(const nvq_grid* grid, const nvq_iso_camera* camera, int persistent, float* image,
@@ -772,7 +809,7 @@ int nvq_fog_march(const nvq_grid* grid, const float* eye, const float* dir, uint
     TileOrder to;
     SlotMap M;
     if (tileOrder(grid->view, eye, dir, sc, to, S(stream), 0, &M) != 0) return NVQ_ERR_HIP;
-    return launchTyped<RunFogMarch>(grid->view.type, grid->view, to.map ? &M : nullptr, eye, dir, sc, to.order, dt,
+    return launchTyped<RunFogMarch>(grid->view.type, grid->view, grid->dview, to.map ? &M : nullptr, eye, dir, sc, to.order, dt,
                                     sigma_t, radiance, transmittance, S(stream));
 }
 

@@ -8,37 +8,29 @@ namespace nvq {
 // Batched ray query: Ray::worldToIndexF (math/Ray.h:258-268), isoCrossing, and the normal from
 // the trilinear gradient at ray(t), Grid::indexToWorldGradF (Map::applyIJTF,
 // math/Math.h:1758-1763), normalised.  v is the value at the hit voxel minus iso.
-template<uint32_t GT>
-__device__ __forceinline__ void zeroCrossingRay(const GridView& g, const float* __restrict__ eye,
-                                                const float* __restrict__ dir, uint64_t i, float iso,
-                                                uint8_t* __restrict__ hit, int32_t* __restrict__ ijk,
-                                                float* __restrict__ tout, float* __restrict__ vout,
-                                                float* __restrict__ normal)
+struct CrossingOut {
+    uint8_t* hit;
+    int32_t* ijk;
+    float *t, *v, *normal;
+};
+
+// Writes ray i's outputs; C holds the corners of the cell at ray(t) where a normal is wanted.
+__device__ __forceinline__ void storeCrossing(const CrossingOut& o, const GridView& g, uint64_t i, bool found,
+                                              const int32_t c[3], float v, float t, const float p[3], const Cell& C)
 {
-    Accessor<GT> acc(g);
-    const float e[3] = {eye[3 * i], eye[3 * i + 1], eye[3 * i + 2]};
-    const float d[3] = {dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]};
-    Ray ray = worldToIndexRay(g, e, d);
-    int32_t c[3] = {0, 0, 0};
-    float v = 0.0f, t = 0.0f;
-    const bool found = isoCrossingCore<GT>(acc, g, ray, iso, c, v, t);
-    if (hit) hit[i] = found ? 1 : 0;
-    if (ijk) {
-        ijk[3 * i] = found ? c[0] : 0;
-        ijk[3 * i + 1] = found ? c[1] : 0;
-        ijk[3 * i + 2] = found ? c[2] : 0;
+    if (o.hit) o.hit[i] = found ? 1 : 0;
+    if (o.ijk) {
+        o.ijk[3 * i] = found ? c[0] : 0;
+        o.ijk[3 * i + 1] = found ? c[1] : 0;
+        o.ijk[3 * i + 2] = found ? c[2] : 0;
     }
-    if (tout) tout[i] = found ? t : 0.0f;
-    if (vout) vout[i] = found ? v : 0.0f;
-    if (normal) {
+    if (o.t) o.t[i] = found ? t : 0.0f;
+    if (o.v) o.v[i] = found ? v : 0.0f;
+    if (o.normal) {
         float nr[3] = {0.0f, 0.0f, 0.0f};
         if (found) {
-            float p[3], gi[3], gw[3];
-            rayAt(ray, t, p);
-            const float fx = floorf(p[0]), fy = floorf(p[1]), fz = floorf(p[2]);
-            Cell C;
-            stencil8(acc, int32_t(fx), int32_t(fy), int32_t(fz), C);
-            trilinearGradient(C, p[0] - fx, p[1] - fy, p[2] - fz, gi);
+            float gi[3], gw[3];
+            trilinearGradient(C, p[0] - floorf(p[0]), p[1] - floorf(p[1]), p[2] - floorf(p[2]), gi);
 #pragma unroll
             for (int a = 0; a < 3; ++a)
                 gw[a] = __builtin_fmaf(gi[0], g.invMatF[a], __builtin_fmaf(gi[1], g.invMatF[3 + a], gi[2] * g.invMatF[6 + a]));
@@ -50,10 +42,52 @@ __device__ __forceinline__ void zeroCrossingRay(const GridView& g, const float* 
                 nr[2] = sc * gw[2];
             }
         }
-        normal[3 * i] = nr[0];
-        normal[3 * i + 1] = nr[1];
-        normal[3 * i + 2] = nr[2];
+        o.normal[3 * i] = nr[0];
+        o.normal[3 * i + 1] = nr[1];
+        o.normal[3 * i + 2] = nr[2];
     }
+}
+
+template<uint32_t GT>
+__device__ __forceinline__ void zeroCrossingRay(const GridView& g, const float* __restrict__ eye,
+                                                const float* __restrict__ dir, uint64_t i, float iso,
+                                                const CrossingOut& o)
+{
+    Accessor<GT> acc(g);
+    const float e[3] = {eye[3 * i], eye[3 * i + 1], eye[3 * i + 2]};
+    const float d[3] = {dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]};
+    Ray ray = worldToIndexRay(g, e, d);
+    int32_t c[3] = {0, 0, 0};
+    float v = 0.0f, t = 0.0f, p[3] = {0.0f, 0.0f, 0.0f};
+    Cell C{};
+    const bool found = isoCrossingCore<GT>(acc, g, ray, iso, c, v, t);
+    if (found && o.normal) {
+        rayAt(ray, t, p);
+        stencil8(acc, ifloor(p[0]), ifloor(p[1]), ifloor(p[2]), C);
+    }
+    storeCrossing(o, g, i, found, c, v, t, p, C);
+}
+
+// The same over a slot map; false, with nothing written, when the map leaves the ray open.
+__device__ __forceinline__ bool zeroCrossingSlots(const SlotMap& M, const GridView& g, const float* __restrict__ eye,
+                                                  const float* __restrict__ dir, uint64_t i, float iso,
+                                                  const CrossingOut& o)
+{
+    const float e[3] = {eye[3 * i], eye[3 * i + 1], eye[3 * i + 2]};
+    const float d[3] = {dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]};
+    Ray ray = worldToIndexRay(g, e, d);
+    int32_t c[3] = {0, 0, 0};
+    float v = 0.0f, t = 0.0f, p[3] = {0.0f, 0.0f, 0.0f};
+    Cell C{};
+    bool open = false;
+    const bool found = isoCrossingSlots(M, g, ray, iso, c, v, t, open);
+    if (open) return false;
+    if (found && o.normal) {
+        rayAt(ray, t, p);
+        if (!slotCorners(M, g, ifloor(p[0]), ifloor(p[1]), ifloor(p[2]), C)) return false;
+    }
+    storeCrossing(o, g, i, found, c, v, t, p, C);
+    return true;
 }
 
 // ------------------------------------------------------------------ fog march

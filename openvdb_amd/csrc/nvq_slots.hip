@@ -1,6 +1,7 @@
 // Slot maps (nvq_slots.h): the flattened view of a grid that the ray queries read.
 //   k_slot_entries : one tree walk per 8^3 slot of the bbox
-//   k_slot_bricks  : one wavefront per leaf decodes its 9^3 brick
+//   k_slot_bricks  : one wavefront per leaf decodes its 9^3 brick (marches)
+//   k_slot_signs   : one wavefront per leaf sets its active and sign bits (crossings)
 #include "nvq_slots.h"
 #include "nvq_internal.h"
 #include "nvq_profile.h"
@@ -13,6 +14,7 @@ namespace nvq {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr uint64_t kSignBytes = 256; // per leaf
 
 template<uint32_t GT>
 __global__ __launch_bounds__(kThreads) void k_slot_entries(GridView g, SlotMap M, uint32_t count,
@@ -29,7 +31,7 @@ __global__ __launch_bounds__(kThreads) void k_slot_entries(GridView g, SlotMap M
     const Probe p = acc.probe((M.lo[0] + int32_t(x)) << 3, (M.lo[1] + int32_t(y)) << 3, (M.lo[2] + int32_t(z)) << 3);
     uint32_t e;
     if (!p.leaf) {
-        e = kSlotTile | (p.active ? kSlotTileOn : 0u) | (p.dim == 8u ? 0u : (p.dim == 128u ? 1u : 2u));
+        e = kSlotTile | (p.active ? kSlotTileOn : 0u) | (p.dim == 8u ? 3u : (p.dim == 128u ? 7u : 12u));
     } else if (p.dim != 1u || x + 1u >= M.n[0] || y + 1u >= M.n[1] || z + 1u >= M.n[2]) {
         e = kSlotOther;
     } else {
@@ -151,6 +153,49 @@ __global__ __launch_bounds__(kThreads) void k_slot_bricks(GridView g, SlotMap M,
     }
 }
 
+// One wavefront per leaf.  Lane l takes byte l % 8 of block l / 8: voxels x & 3 = k / 2, y & 3 =
+// 2 (k & 1) + {0, 1}, z & 3 = 0..3, as two rows of four.
+template<uint32_t GT>
+__global__ __launch_bounds__(kThreads) void k_slot_signs(GridView g, SlotMap M, uint32_t count,
+                                                         const uint32_t* __restrict__ slotOf, float iso,
+                                                         uint8_t* __restrict__ signs)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t b = __builtin_amdgcn_readfirstlane(blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6));
+    if (b >= g.leafCount) return;
+    const uint32_t slot = __builtin_amdgcn_readfirstlane(slotOf[b]);
+    if (slot >= count || M.entry[slot] != b) return; // as in k_slot_bricks
+    const uint8_t* leaf = g.leaf0 + (GT == GT_FPN ? uint64_t(M.leafOff[b]) << 5 : uint64_t(b) * g.leafSize);
+    const uint32_t block = lane >> 3, k = lane & 7u;
+    const uint32_t x = (block >> 2) * 4u + (k >> 1), y = ((block >> 1) & 1u) * 4u + (k & 1u) * 2u, z = (block & 1u) * 4u;
+    const uint64_t word = ld_u64(leaf + kLeafVMask + 8u * x);
+    uint32_t on = 0, below = 0, above = 0;
+#pragma unroll
+    for (uint32_t r = 0; r < 2; ++r) {
+        const uint32_t n = (x << 6) | ((y + r) << 3) | z;
+        on |= (uint32_t(word >> ((y + r) * 8u + z)) & 15u) << (4u * r);
+        float v[4];
+        if constexpr (GT == GT_FLOAT) {
+            const float4 f = *reinterpret_cast<const float4*>(leaf + kLeafData + 4u * n);
+            v[0] = f.x; v[1] = f.y; v[2] = f.z; v[3] = f.w;
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) v[j] = Codec<GT>::get(leaf, n + j, g.channel);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const float d = v[j] - iso;
+            below |= (d < 0.0f ? 1u : 0u) << (4u * r + j);
+            above |= (d > 0.0f ? 1u : 0u) << (4u * r + j);
+        }
+    }
+    uint8_t* out = signs + (uint64_t(b) * 8u + block) * 32u + k;
+    out[0] = uint8_t(on);
+    out[8] = uint8_t(below);
+    out[16] = uint8_t(on);
+    out[24] = uint8_t(above);
+}
+
 __global__ void k_zero_word(uint32_t* p) { *p = 0u; }
 
 bool slotBox(const GridView& g, int32_t lo[3], uint32_t n[3], uint64_t& count)
@@ -172,19 +217,22 @@ size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
 template<uint32_t GT>
 void launchMap(const GridView& g, const SlotMap& M, uint32_t count, uint32_t* entry, float* value, uint32_t* tileIndex,
-               float* brick, uint32_t* slotOf, uint32_t* leafOff, uint32_t* leaves, hipStream_t s)
+               float* brick, uint8_t* signs, float iso, uint32_t* slotOf, uint32_t* leafOff, uint32_t* leaves,
+               hipStream_t s)
 {
     if (GT == GT_FPN) hipLaunchKernelGGL(k_zero_word, dim3(1), dim3(1), 0, s, leaves);
     hipLaunchKernelGGL(k_slot_entries<GT>, dim3((count + kThreads - 1) / kThreads), dim3(kThreads), 0, s, g, M, count,
                        entry, value, tileIndex, slotOf, leafOff, leaves);
-    if (g.leafCount)
-        hipLaunchKernelGGL(k_slot_bricks<GT>, dim3((g.leafCount + kThreads / 64 - 1) / (kThreads / 64)), dim3(kThreads), 0,
-                           s, g, M, count, slotOf, leafOff, brick);
+    const dim3 waves((g.leafCount + kThreads / 64 - 1) / (kThreads / 64));
+    if (g.leafCount && brick)
+        hipLaunchKernelGGL(k_slot_bricks<GT>, waves, dim3(kThreads), 0, s, g, M, count, slotOf, leafOff, brick);
+    if (g.leafCount && signs)
+        hipLaunchKernelGGL(k_slot_signs<GT>, waves, dim3(kThreads), 0, s, g, M, count, slotOf, iso, signs);
 }
 
 } // namespace
 
-size_t slotMapBytes(const GridView& g, uint64_t rays)
+size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts)
 {
     int32_t lo[3];
     uint32_t n[3];
@@ -195,10 +243,10 @@ size_t slotMapBytes(const GridView& g, uint64_t rays)
         return 0;
     const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
     return up256(4 * count) * (g.type == GT_ONINDEX ? 3 : 2) + up256(4 * leaves) * 2 + 256 +
-           up256(4ull * kBrickFloats * leaves);
+           (parts & kMapBricks ? up256(4ull * kBrickFloats * leaves) : 0) + (parts & kMapSigns ? up256(kSignBytes * leaves) : 0);
 }
 
-int launchSlotMap(const GridView& g, char* mem, SlotMap& M, hipStream_t s)
+int launchSlotMap(const GridView& g, char* mem, SlotMap& M, uint32_t parts, float iso, hipStream_t s)
 {
     uint64_t count;
     if (!slotBox(g, M.lo, M.n, count)) return -1;
@@ -215,20 +263,23 @@ int launchSlotMap(const GridView& g, char* mem, SlotMap& M, hipStream_t s)
     uint32_t* slotOf = reinterpret_cast<uint32_t*>(take(4 * leaves));
     uint32_t* leafOff = reinterpret_cast<uint32_t*>(take(4 * leaves));
     uint32_t* number = reinterpret_cast<uint32_t*>(take(4));
-    float* brick = reinterpret_cast<float*>(take(4ull * kBrickFloats * leaves));
+    float* brick = parts & kMapBricks ? reinterpret_cast<float*>(take(4ull * kBrickFloats * leaves)) : nullptr;
+    uint8_t* signs = parts & kMapSigns ? reinterpret_cast<uint8_t*>(take(kSignBytes * leaves)) : nullptr;
     M.entry = entry;
     M.value = value;
     M.brick = brick;
     M.tileIndex = index;
+    M.signs = reinterpret_cast<const uint4*>(signs);
+    M.leafOff = leafOff;
     ProfScope prof("slot_map", s);
     const uint32_t c = uint32_t(count);
     switch (g.type) {
-    case GT_FLOAT: launchMap<GT_FLOAT>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
-    case GT_FP4: launchMap<GT_FP4>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
-    case GT_FP8: launchMap<GT_FP8>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
-    case GT_FP16: launchMap<GT_FP16>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
-    case GT_FPN: launchMap<GT_FPN>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
-    case GT_ONINDEX: launchMap<GT_ONINDEX>(g, M, c, entry, value, index, brick, slotOf, leafOff, number, s); break;
+    case GT_FLOAT: launchMap<GT_FLOAT>(g, M, c, entry, value, index, brick, signs, iso, slotOf, leafOff, number, s); break;
+    case GT_FP4: launchMap<GT_FP4>(g, M, c, entry, value, index, brick, signs, iso, slotOf, leafOff, number, s); break;
+    case GT_FP8: launchMap<GT_FP8>(g, M, c, entry, value, index, brick, signs, iso, slotOf, leafOff, number, s); break;
+    case GT_FP16: launchMap<GT_FP16>(g, M, c, entry, value, index, brick, signs, iso, slotOf, leafOff, number, s); break;
+    case GT_FPN: launchMap<GT_FPN>(g, M, c, entry, value, index, brick, signs, iso, slotOf, leafOff, number, s); break;
+    case GT_ONINDEX: launchMap<GT_ONINDEX>(g, M, c, entry, value, index, brick, signs, iso, slotOf, leafOff, number, s); break;
     default: return -3;
     }
     return hipGetLastError() == hipSuccess ? 0 : -4;

@@ -1,5 +1,5 @@
-"""The fog march over a slot map against the same march through the accessor, bit for bit, and its
-adjoint (2x2x2 blocks in LDS) against the FP64 oracle and across schedules and grid types.
+"""The fog march and the level-set crossings over a slot map against the same queries through the
+accessor, bit for bit, and the march's adjoint (2x2x2 blocks in LDS) against the FP64 oracle and across schedules and grid types.
 
 A launch under graph capture takes no scratch and goes through the accessor, so a captured call is
 the reference here; the march itself is compared with the FP64 oracle in test_gpu_parity.py.
@@ -87,6 +87,40 @@ def test_march_over_slots_equals_march_through_the_accessor(name, codec):
             assert torch.equal(L, L2)
         if n > 64:
             assert float(L.max()) > 0.0
+
+
+def _level_set(nvq, name):
+    if name == "torus":
+        return nvq.tools.create_level_set_torus(50.0, 14.0, (3.0, -2.0, 5.0), 0.5, 3.0)
+    if name == "tiles":
+        return _host(nvq, "tiles")  # active tiles: candidates outside leaves
+    sphere = nvq.tools.create_level_set_sphere(37.0, (1.5, -2.0, 3.0), 1.0, 3.0)
+    return _flagged(sphere) if name == "flagged" else sphere
+
+
+@pytest.mark.parametrize("name,codec", [("sphere", c) for c in ("float", "fp4", "fp8", "fp16", "fpn")] +
+                         [("torus", "float"), ("torus", "fpn"), ("tiles", "float"), ("flagged", "float")])
+def test_crossing_over_slots_equals_crossing_through_the_accessor(name, codec):
+    nvq = _nvq()
+    d = _grid(nvq, _level_set(nvq, name), codec)
+    for n, iso in ((1, 0.0), (65, 0.0), (20011, 0.0), (20011, 0.4), (4097, -0.7)):
+        eye, dirs = _rays(d, n)
+        eye *= d.voxel_size[0]
+        got = nvq.ops.iso_crossing(d, eye, dirs, iso)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            want = nvq.ops.iso_crossing(d, eye, dirs, iso)
+        for _ in range(2):
+            for x in want:
+                x.fill_(7)
+            graph.replay()
+            torch.cuda.synchronize()
+            for a, b in zip(got, want):
+                assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), (n, iso)
+            nvq.ops.iso_crossing(d, eye, dirs, iso)
+        if n > 4096 and iso == 0.0 and name != "tiles":
+            assert int(got[0].sum()) > 1000
 
 
 @pytest.fixture(scope="module")
