@@ -7,8 +7,8 @@
 //                    background value of slots without a leaf
 //   k_bin_classify : per query, whether a slot of its [cell-1, cell+2]^3 block holds a leaf (map
 //                    staged in LDS); marks those queries per chunk of 2048 and counts them
-//   scan + compact : the marked queries' bin keys (16^3 bins over the grid's active bbox grown by
-//                    2 voxels; points outside are clamped into the border bins) and points
+//   scan + compact : the marked queries' bin keys (16^3 bins over the leaves of the grid's active
+//                    bbox grown by 2 voxels; points outside are clamped into the border bins) and points
 //                    {index-space xyz, original index}, in chunk order; the call waits once, to
 //                    size the sort
 //   radix sort     : (key, point) pairs of the marked queries (rocPRIM/hipCUB DeviceRadixSort)
@@ -576,19 +576,17 @@ __global__ __launch_bounds__(kThreads) void k_sample_list(GridView g, const floa
                                                           const uint32_t* __restrict__ count, Rec* __restrict__ rec,
                                                           bool wantNN, bool wantVal, int mode, SampleConsts k)
 {
-    Accessor<GT> acc(g);
     const uint32_t m = *count;
     for (uint32_t base = blockIdx.x * kThreads + (threadIdx.x & ~63u); base < m; base += gridDim.x * kThreads) {
         const uint32_t j = base + (threadIdx.x & 63u);
         const bool valid = j < m;
-        SampleOut r{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
         uint32_t id = 0;
+        float p[3] = {0.0f, 0.0f, 0.0f};
         if (valid) {
             id = list[j];
-            float p[3];
             loadPoint(g, xyz, id, world, p);
-            r = sampleEval(acc, p, wantNN, wantVal, mode, k);
         }
+        const SampleOut r = sampleWave<GT>(g, valid, p, wantNN, wantVal, mode, k);
         storeRecQuad(rec, valid, id, r.nn, r.val, r.g);
     }
 }
@@ -719,15 +717,16 @@ __global__ __launch_bounds__(kThreads) void k_sample_bwd(GridView g, const float
                                                          float scale, unsigned long long* __restrict__ accum,
                                                          uint32_t* __restrict__ overflow)
 {
-    Accessor<GT> acc(g);
     bool ok = true;
     const uint64_t stride = uint64_t(gridDim.x) * kThreads;
-    for (uint64_t i = uint64_t(blockIdx.x) * kThreads + threadIdx.x; i < n; i += stride) {
-        const SampleGrad d = loadGrad(gnn, gval, ggrad, i);
-        if (gradZero(d)) continue;
-        float p[3];
-        loadPoint(g, xyz, i, world, p);
-        sampleAdjointOne(acc, g, p, d, mode, k, scale, accum, ok);
+    for (uint64_t base = uint64_t(blockIdx.x) * kThreads + (threadIdx.x & ~63u); base < n; base += stride) {
+        const uint64_t i = base + (threadIdx.x & 63u);
+        SampleGrad d{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
+        if (i < n) d = loadGrad(gnn, gval, ggrad, i);
+        const bool valid = i < n && !gradZero(d);
+        float p[3] = {0.0f, 0.0f, 0.0f};
+        if (valid) loadPoint(g, xyz, i, world, p);
+        sampleAdjointLanes<GT>(g, valid, p, d, mode, k, scale, accum, ok);
     }
     if (!ok) atomicOr(overflow, 1u);
 }
@@ -744,14 +743,19 @@ __global__ __launch_bounds__(kThreads) void k_sample_bwd_list(GridView g, const 
                                                               unsigned long long* __restrict__ accum,
                                                               uint32_t* __restrict__ overflow)
 {
-    Accessor<GT> acc(g);
     bool ok = true;
     const uint32_t m = *count;
-    for (uint32_t j = blockIdx.x * kThreads + threadIdx.x; j < m; j += gridDim.x * kThreads) {
-        const uint32_t id = list[j];
-        float p[3];
-        loadPoint(g, xyz, id, world, p);
-        sampleAdjointOne(acc, g, p, loadGrad(gnn, gval, ggrad, id), mode, k, scale, accum, ok);
+    for (uint32_t base = blockIdx.x * kThreads + (threadIdx.x & ~63u); base < m; base += gridDim.x * kThreads) {
+        const uint32_t j = base + (threadIdx.x & 63u);
+        const bool valid = j < m;
+        float p[3] = {0.0f, 0.0f, 0.0f};
+        SampleGrad d{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
+        if (valid) {
+            const uint32_t id = list[j];
+            loadPoint(g, xyz, id, world, p);
+            d = loadGrad(gnn, gval, ggrad, id);
+        }
+        sampleAdjointLanes<GT>(g, valid, p, d, mode, k, scale, accum, ok);
     }
     if (!ok) atomicOr(overflow, 1u);
 }
@@ -843,7 +847,9 @@ bool makeLayout(const GridView& g, BinLayout& L)
     if (g.bbox[0] > g.bbox[3] || g.bbox[1] > g.bbox[4] || g.bbox[2] > g.bbox[5]) return false; // empty grid
     uint64_t total = 1;
     for (int a = 0; a < 3; ++a) {
-        const int64_t lo = int64_t(g.bbox[a]) - 2, hi = int64_t(g.bbox[3 + a]) + 2;
+        // whole leaves and two voxels more: points in a leaf that reaches past the bbox of the active voxels
+        // would otherwise leave their brick and go through the lane kernel one by one
+        const int64_t lo = (int64_t(g.bbox[a]) & ~int64_t(7)) - 2, hi = (int64_t(g.bbox[3 + a]) | 7) + 2;
         const int64_t nb = ((hi - lo) >> kBinLog2) + 1;
         if (nb > (int64_t(1) << 20)) return false;
         L.lo[a] = int32_t(lo);

@@ -126,20 +126,328 @@ __device__ __forceinline__ SampleOut sampleEval(Accessor<GT>& acc, const float p
     return r;
 }
 
-// Evaluate one query at index-space p; writes the requested outputs at index i.
-template<uint32_t GT>
-__device__ __forceinline__ void sampleOne(Accessor<GT>& acc, const float p[3], uint64_t i, float* __restrict__ nn,
-                                          float* __restrict__ val, float* __restrict__ grad, int mode,
-                                          const SampleConsts& k)
+// The six FD6 sample points of the forward (sampleEval): p + (+-1 along one axis, +-0 on the others)
+__host__ __device__ __forceinline__ void fd6Points(const float p[3], float q[6][3])
 {
-    const SampleOut r = sampleEval(acc, p, nn != nullptr, val != nullptr, grad ? mode : 0, k);
-    if (nn) nn[i] = r.nn;
-    if (val) val[i] = r.val;
-    if (grad) {
-        grad[3 * i] = r.g[0];
-        grad[3 * i + 1] = r.g[1];
-        grad[3 * i + 2] = r.g[2];
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+        const int ax = t >> 1;
+        const bool plus = (t & 1) == 0;
+#pragma unroll
+        for (int b = 0; b < 3; ++b) {
+            const float dlt = b == ax ? 1.0f : 0.0f;
+            q[t][b] = plus ? p[b] + dlt : p[b] - dlt;
+        }
     }
+}
+
+// True when every voxel the query's terms reach lies in the plus-shaped block around its cell
+// (cell + [-1, 2] on one axis, cell + [0, 1] on the others): always, except for FD6 sample points
+// whose p +- 1 rounds into a cell other than the neighbouring one.
+__host__ __device__ __forceinline__ bool adjointInBlock(const float p[3], int mode)
+{
+    if (mode != 1) return true;
+    float q[6][3];
+    fd6Points(p, q);
+    bool ok = true;
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+        const int ax = t >> 1;
+        const float expect = floorf(p[ax]) + ((t & 1) ? -1.0f : 1.0f);
+        ok = ok && floorf(q[t][ax]) == expect;
+    }
+    return ok;
+}
+
+// ------------------------------------------------------------------ staged queries
+// The 8^3 slots that the block [cell-1, cell+2]^3 of a query overlaps (one or two per axis), resolved
+// to their leaf or tile value in four stages (root, upper, lower, voxels), every load of a stage in
+// flight at once.  Through the accessor each of the up to 32 voxels is its own guarded lookup and the
+// lookups wait for each other: 1000 queries took 61 us, 300,007 took 163 us.
+constexpr uint32_t kNoLeaf = 0xffffffffu;
+struct BlockSlots {
+    int32_t s0[3];    // first slot per axis
+    uint32_t leaf[8]; // offset from leaf0 in units of 32 bytes, or kNoLeaf; slot (a, b, c) at 4a + 2b + c
+    float tile[8];    // value of a slot without a leaf
+    uint32_t index[8]; // index grids: its channel index
+};
+
+// False where the query goes through the accessor: a cell near the ends of the integer range, or leaves
+// beyond the 32-bit offsets.  `keys`: fill index[].
+template<uint32_t GT>
+__device__ __forceinline__ bool resolveBlock(const GridView& g, int32_t i0, int32_t j0, int32_t k0, bool keys, BlockSlots& B)
+{
+    const int32_t cell[3] = {i0, j0, k0};
+    bool two[3], ok = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        ok = ok && cell[a] > -(1 << 30) && cell[a] < (1 << 30);
+        B.s0[a] = (cell[a] - 1) >> 3;
+        const int32_t s1 = (cell[a] + 2) >> 3;
+        two[a] = s1 != B.s0[a];
+    }
+    if (!ok) return false;
+    auto need = [&](int s) { return (!(s & 4) || two[0]) && (!(s & 2) || two[1]) && (!(s & 1) || two[2]); };
+    // root: the tile of each slot (a grid around the origin has one per octant)
+    uint32_t part[3][2], tile[8], missing = 0; // tile: its number + 1, or 0
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) part[a][b] = uint32_t((B.s0[a] + b) << 3) >> 12;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        tile[s] = 0;
+        missing += need(s) ? 1u : 0u;
+    }
+    for (uint32_t i = 0; i < g.tableSize && missing; ++i) { // uniform addresses: scalar loads
+        const uint64_t key = ld_u64(g.root + rootHeaderSize(GT) + kTileSize * i);
+        const uint32_t kx = uint32_t(key >> 42), ky = uint32_t(key >> 21) & 0x1fffffu, kz = uint32_t(key) & 0x1fffffu;
+        const bool x[2] = {part[0][0] == kx, part[0][1] == kx}, y[2] = {part[1][0] == ky, part[1][1] == ky},
+                   z[2] = {part[2][0] == kz, part[2][1] == kz};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const bool is = x[s >> 2] && y[(s >> 1) & 1] && z[s & 1] && need(s) && tile[s] == 0; // the first match
+            tile[s] = is ? i + 1u : tile[s];
+            missing -= is ? 1u : 0u;
+        }
+    }
+    const uint8_t* node[8];
+    uint64_t entry[8]; // float bits or channel index of a slot that ends at the current level
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        node[s] = nullptr;
+        entry[s] = 0;
+        B.leaf[s] = kNoLeaf;
+    }
+    const uint64_t background =
+        GT == GT_ONINDEX ? ld_u64(g.root + kIdxRootBackground) : uint64_t(__float_as_uint(g.background));
+    {
+        uint32_t mask[8];
+        uint64_t e[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            mask[s] = 0;
+            entry[s] = background;
+            e[s] = 0;
+            if (!need(s) || tile[s] == 0) continue;
+            const uint8_t* t = g.root + rootHeaderSize(GT) + kTileSize * (tile[s] - 1u);
+            e[s] = ld_u64(t + 8);
+            entry[s] = GT == GT_ONINDEX ? ld_u64(t + kIdxTileValue) : uint64_t(ld_u32(t + 20));
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+            if (e[s]) node[s] = g.root + int64_t(e[s]);
+        // upper
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (!node[s]) continue;
+            const uint32_t x = uint32_t(B.s0[0] + (s >> 2)), y = uint32_t(B.s0[1] + ((s >> 1) & 1)), z = uint32_t(B.s0[2] + (s & 1));
+            const uint32_t n = (((x & 511u) >> 4) << 10) | (((y & 511u) >> 4) << 5) | ((z & 511u) >> 4);
+            mask[s] = maskOn(node[s] + kUpCMask, n) ? 1u : 0u;
+            e[s] = ld_u64(node[s] + kUpTable + 8 * n);
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (!node[s]) continue;
+            entry[s] = e[s];
+            node[s] = mask[s] ? node[s] + int64_t(e[s]) : nullptr;
+        }
+        // lower
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            mask[s] = 0;
+            e[s] = 0;
+            if (!node[s]) continue;
+            const uint32_t x = uint32_t(B.s0[0] + (s >> 2)), y = uint32_t(B.s0[1] + ((s >> 1) & 1)), z = uint32_t(B.s0[2] + (s & 1));
+            const uint32_t n = ((x & 15u) << 8) | ((y & 15u) << 4) | (z & 15u);
+            mask[s] = maskOn(node[s] + kLoCMask, n) ? 1u : 0u;
+            e[s] = ld_u64(node[s] + kLoTable + 8 * n);
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (!node[s]) continue;
+            if (mask[s]) {
+                const uint64_t off = uint64_t(node[s] + int64_t(e[s]) - g.leaf0);
+                ok = ok && (off & 31u) == 0 && off < (uint64_t(kNoLeaf) << 5);
+                B.leaf[s] = uint32_t(off >> 5);
+            } else {
+                entry[s] = e[s];
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        if constexpr (GT == GT_ONINDEX) {
+            B.index[s] = uint32_t(entry[s]);
+            B.tile[s] = 0.0f;
+            if (!keys && need(s) && B.leaf[s] == kNoLeaf) B.tile[s] = g.channel[entry[s]];
+        } else {
+            B.tile[s] = __uint_as_float(uint32_t(entry[s]));
+        }
+    }
+    return ok;
+}
+
+// The slot of voxel (x, y, z) of the block, its entries chosen without dynamic indexing.
+template<class T>
+__device__ __forceinline__ T pickSlot(const BlockSlots& B, const T (&v)[8], int32_t x, int32_t y, int32_t z)
+{
+    T v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3], v4 = v[4], v5 = v[5], v6 = v[6], v7 = v[7];
+    asm("" : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3), "+v"(v4), "+v"(v5), "+v"(v6), "+v"(v7));
+    const bool a = (x >> 3) != B.s0[0], b = (y >> 3) != B.s0[1], c = (z >> 3) != B.s0[2];
+    const T w0 = a ? v4 : v0, w1 = a ? v5 : v1, w2 = a ? v6 : v2, w3 = a ? v7 : v3;
+    const T u0 = b ? w2 : w0, u1 = b ? w3 : w1;
+    return c ? u1 : u0;
+}
+
+template<uint32_t GT>
+__device__ __forceinline__ float blockVoxel(const GridView& g, const BlockSlots& B, int32_t x, int32_t y, int32_t z)
+{
+    const uint32_t leaf = pickSlot(B, B.leaf, x, y, z);
+    float v = pickSlot(B, B.tile, x, y, z);
+    if (leaf != kNoLeaf) v = Codec<GT>::get(g.leaf0 + (uint64_t(leaf) << 5), Accessor<GT>::leafOffset(x, y, z), g.channel);
+    return v;
+}
+
+// sampleEval over resolved slots, with its operations in its order, for queries whose FD6 cells are the
+// neighbouring ones (adjointInBlock).  False: through the accessor.
+template<uint32_t GT>
+__device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3], bool wantNN, bool wantVal, int mode,
+                                             const SampleConsts& k, SampleOut& r)
+{
+    const float fx = floorf(p[0]), fy = floorf(p[1]), fz = floorf(p[2]);
+    const int32_t i0 = int32_t(fx), j0 = int32_t(fy), k0 = int32_t(fz);
+    const int32_t ri = int32_t(rintf(p[0])) - i0, rj = int32_t(rintf(p[1])) - j0, rk = int32_t(rintf(p[2])) - k0;
+    BlockSlots B;
+    if (((ri | rj | rk) & ~1) || !resolveBlock<GT>(g, i0, j0, k0, false, B)) return false;
+    const float u = p[0] - fx, v = p[1] - fy, w = p[2] - fz;
+    Cell C;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) C.v[a][b][e] = blockVoxel<GT>(g, B, i0 + a, j0 + b, k0 + e);
+    r = SampleOut{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
+    if (mode == 1) {
+        // the layers next to the cell: [axis][side][the other two axes]
+        float L[3][2][2][2];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) {
+                    L[0][s][a][b] = blockVoxel<GT>(g, B, i0 + (s ? 2 : -1), j0 + a, k0 + b);
+                    L[1][s][a][b] = blockVoxel<GT>(g, B, i0 + a, j0 + (s ? 2 : -1), k0 + b);
+                    L[2][s][a][b] = blockVoxel<GT>(g, B, i0 + a, j0 + b, k0 + (s ? 2 : -1));
+                }
+        if (wantNN) r.nn = pick(C, ri, rj, rk);
+        if (wantVal) r.val = trilerp(C, u, v, w);
+        float f[3][2];
+#pragma unroll
+        for (int axis = 0; axis < 3; ++axis)
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                Cell D;
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        // near and far face of the neighbouring cell along the axis
+                        const float edge = L[axis][s][a][b];
+                        const float face = axis == 0 ? C.v[s][a][b] : (axis == 1 ? C.v[a][s][b] : C.v[a][b][s]);
+                        const float lo = s ? face : edge, hi = s ? edge : face;
+                        if (axis == 0) { D.v[0][a][b] = lo; D.v[1][a][b] = hi; }
+                        if (axis == 1) { D.v[a][0][b] = lo; D.v[a][1][b] = hi; }
+                        if (axis == 2) { D.v[a][b][0] = lo; D.v[a][b][1] = hi; }
+                    }
+                const float d = s ? 1.0f : -1.0f;
+                const float qx = axis == 0 ? p[0] + d : p[0] + 0.0f, qy = axis == 1 ? p[1] + d : p[1] + 0.0f,
+                            qz = axis == 2 ? p[2] + d : p[2] + 0.0f;
+                f[axis][s] = trilerp(D, qx - floorf(qx), qy - floorf(qy), qz - floorf(qz));
+            }
+        r.g[0] = (f[0][1] - f[0][0]) * k.fdx;
+        r.g[1] = (f[1][1] - f[1][0]) * k.fdy;
+        r.g[2] = (f[2][1] - f[2][0]) * k.fdz;
+        return true;
+    }
+    if (wantNN) r.nn = pick(C, ri, rj, rk);
+    if (wantVal) r.val = trilerp(C, u, v, w);
+    if (mode == 2) {
+        const float mx = blockVoxel<GT>(g, B, i0 - 1, j0, k0), my = blockVoxel<GT>(g, B, i0, j0 - 1, k0),
+                    mz = blockVoxel<GT>(g, B, i0, j0, k0 - 1);
+        r.g[0] = k.gsInv2dx * (C.v[1][0][0] - mx);
+        r.g[1] = k.gsInv2dx * (C.v[0][1][0] - my);
+        r.g[2] = k.gsInv2dx * (C.v[0][0][1] - mz);
+    } else if (mode == 3) {
+        trilinearGradient(C, u, v, w, r.g);
+    }
+    return true;
+}
+
+// FD6 queries whose p +- 1 rounds into a farther cell, about one in a million: the wavefront evaluates
+// them one after the other, lane 8 t + c fetching corner c of sample t (0: the value, 1..6: +x, -x, +y,
+// -y, +z, -z) and lane 56 the nearest voxel.  One such lane going through sampleEval held its whole
+// wavefront for 60 us.  Every lane of the wavefront calls this; `mine` marks the queries.
+template<uint32_t GT>
+__device__ __forceinline__ void sampleOffBlock(const GridView& g, bool mine, const float p[3], bool wantNN, bool wantVal,
+                                               const SampleConsts& k, SampleOut& r)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint64_t todo = __ballot(mine);
+    while (todo) {
+        const int src = __builtin_ctzll(todo);
+        todo &= todo - 1u;
+        const float P[3] = {__shfl(p[0], src, 64), __shfl(p[1], src, 64), __shfl(p[2], src, 64)};
+        const uint32_t t = lane >> 3, c = lane & 7u;
+        // the forward's own sums: p + (+-1 along one axis, +-0 along the others)
+        float q[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float d = t != 0 && uint32_t(a) == (t - 1u) >> 1 ? 1.0f : 0.0f;
+            q[a] = t == 0 ? P[a] : ((t & 1u) ? P[a] + d : P[a] - d);
+        }
+        const float fx = floorf(q[0]), fy = floorf(q[1]), fz = floorf(q[2]);
+        int32_t x = int32_t(fx) + int32_t(c >> 2), y = int32_t(fy) + int32_t((c >> 1) & 1u), z = int32_t(fz) + int32_t(c & 1u);
+        if (t == 7u) {
+            x = int32_t(rintf(P[0]));
+            y = int32_t(rintf(P[1]));
+            z = int32_t(rintf(P[2]));
+        }
+        Accessor<GT> acc(g);
+        const float v = acc.probe(x, y, z).value;
+        Cell C;
+        const int first = int(lane & ~7u);
+#pragma unroll
+        for (int s = 0; s < 8; ++s) C.v[s >> 2][(s >> 1) & 1][s & 1] = __shfl(v, first + s, 64);
+        const float f = trilerp(C, q[0] - fx, q[1] - fy, q[2] - fz);
+        const float val = __shfl(f, 0, 64), nn = __shfl(v, 56, 64);
+        const float d[3] = {__shfl(f, 8, 64) - __shfl(f, 16, 64), __shfl(f, 24, 64) - __shfl(f, 32, 64),
+                            __shfl(f, 40, 64) - __shfl(f, 48, 64)};
+        if (int(lane) == src) {
+            r.nn = wantNN ? nn : 0.0f;
+            r.val = wantVal ? val : 0.0f;
+            r.g[0] = d[0] * k.fdx;
+            r.g[1] = d[1] * k.fdy;
+            r.g[2] = d[2] * k.fdz;
+        }
+    }
+}
+
+// One query per lane; every lane of the wavefront calls this, `valid` or not.
+template<uint32_t GT>
+__device__ __forceinline__ SampleOut sampleWave(const GridView& g, bool valid, const float p[3], bool wantNN, bool wantVal,
+                                                int mode, const SampleConsts& k)
+{
+    SampleOut r{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
+    const bool off = valid && !adjointInBlock(p, mode);
+    if (valid && !off && !sampleStaged<GT>(g, p, wantNN, wantVal, mode, k, r)) {
+        Accessor<GT> acc(g);
+        r = sampleEval(acc, p, wantNN, wantVal, mode, k);
+    }
+    if (__any(off)) sampleOffBlock<GT>(g, off, p, wantNN, wantVal, k, r);
+    return r;
 }
 
 // ------------------------------------------------------------------ adjoint of the point queries
@@ -175,120 +483,65 @@ __device__ __forceinline__ long long toFixedSat(float x, bool& ok)
     return x > 0.0f ? (1ll << 62) : -(1ll << 62);
 }
 
-struct AdjTerm {
-    int32_t o[3];
-    float s;
-    float A[2], B[2], C[2];
-    bool single;
-};
-
-// The six FD6 sample points of the forward (sampleEval): p + (+-1 along one axis, +-0 on the others)
-__host__ __device__ __forceinline__ void fd6Points(const float p[3], float q[6][3])
-{
-#pragma unroll
-    for (int t = 0; t < 6; ++t) {
-        const int ax = t >> 1;
-        const bool plus = (t & 1) == 0;
-#pragma unroll
-        for (int b = 0; b < 3; ++b) {
-            const float dlt = b == ax ? 1.0f : 0.0f;
-            q[t][b] = plus ? p[b] + dlt : p[b] - dlt;
-        }
-    }
-}
-
-// General form: the query's terms as a list, each voxel's sum formed in term order.  Used when an
-// FD6 sample cell is not the one next to the query's cell (float rounding of p +- 1) and in
-// kernels that must not assume the plus-shaped block.  emit(x, y, z, contribution) once per voxel.
+// General form of the sums, for FD6 sample cells that are not the ones next to the query's cell (float
+// rounding of p +- 1): the whole wavefront takes one query, lane 8 t + c holding corner c of term t.
+// Terms are numbered in the contract's order, so a voxel's sum is that of its lanes in lane order, and
+// its first lane emits it.  (One lane looping over all pairs of corners took 330 us.)
+// emit(x, y, z, contribution).  Every lane calls this with the same query.
 template<class Emit>
-__host__ __device__ __noinline__ void sampleAdjointGeneral(const float p[3], const SampleGrad& d, int mode,
-                                                   const SampleConsts& k, Emit& emit)
+__device__ __forceinline__ void sampleAdjointWave(const float p[3], const SampleGrad& d, int mode, const SampleConsts& k,
+                                                  Emit& emit)
 {
-    AdjTerm T[8];
-    int nt = 0;
+    const uint32_t lane = threadIdx.x & 63u, mine = lane >> 3, c = lane & 7u;
+    uint32_t terms = 0;
+    int32_t x = 0, y = 0, z = 0;
+    float w = 0.0f;
+    bool have = false;
     const float fx = floorf(p[0]), fy = floorf(p[1]), fz = floorf(p[2]);
     const int32_t i0 = int32_t(fx), j0 = int32_t(fy), k0 = int32_t(fz);
-    const float u = p[0] - fx, v = p[1] - fy, w = p[2] - fz;
-    auto cellTerm = [&](int32_t x, int32_t y, int32_t z, float s, float a0, float a1, float b0, float b1, float c0,
+    const float u = p[0] - fx, v = p[1] - fy, t = p[2] - fz;
+    auto cellTerm = [&](int32_t ox, int32_t oy, int32_t oz, float s, float a0, float a1, float b0, float b1, float c0,
                         float c1) {
-        AdjTerm& t = T[nt++];
-        t.o[0] = x; t.o[1] = y; t.o[2] = z;
-        t.s = s;
-        t.A[0] = a0; t.A[1] = a1; t.B[0] = b0; t.B[1] = b1; t.C[0] = c0; t.C[1] = c1;
-        t.single = false;
+        if (terms++ != mine) return;
+        x = ox + int32_t(c >> 2);
+        y = oy + int32_t((c >> 1) & 1u);
+        z = oz + int32_t(c & 1u);
+        w = ((s * ((c & 4u) ? a1 : a0)) * ((c & 2u) ? b1 : b0)) * ((c & 1u) ? c1 : c0);
+        have = true;
     };
-    auto singleTerm = [&](int32_t x, int32_t y, int32_t z, float s) {
-        AdjTerm& t = T[nt++];
-        t.o[0] = x; t.o[1] = y; t.o[2] = z;
-        t.s = s;
-        t.single = true;
-    };
-    if (d.gv != 0.0f) cellTerm(i0, j0, k0, d.gv, 1.0f - u, u, 1.0f - v, v, 1.0f - w, w);
-    if (mode == 1) {
-        float q[6][3];
-        fd6Points(p, q);
-        const float fd[3] = {k.fdx, k.fdy, k.fdz};
-        for (int t = 0; t < 6; ++t) {
-            const float s0 = d.gg[t >> 1] * fd[t >> 1];
-            const float s = (t & 1) ? -s0 : s0;
-            if (s == 0.0f) continue;
-            const float gx = floorf(q[t][0]), gy = floorf(q[t][1]), gz = floorf(q[t][2]);
-            const float a = q[t][0] - gx, b = q[t][1] - gy, c = q[t][2] - gz;
-            cellTerm(int32_t(gx), int32_t(gy), int32_t(gz), s, 1.0f - a, a, 1.0f - b, b, 1.0f - c, c);
-        }
-    } else if (mode == 2) {
-        for (int ax = 0; ax < 3; ++ax) {
-            const float s = k.gsInv2dx * d.gg[ax];
-            if (s == 0.0f) continue;
-            const int32_t dx = ax == 0, dy = ax == 1, dz = ax == 2;
-            singleTerm(i0 + dx, j0 + dy, k0 + dz, s);
-            singleTerm(i0 - dx, j0 - dy, k0 - dz, -s);
-        }
-    } else if (mode == 3) {
-        if (d.gg[0] != 0.0f) cellTerm(i0, j0, k0, d.gg[0], -1.0f, 1.0f, 1.0f - v, v, 1.0f - w, w);
-        if (d.gg[1] != 0.0f) cellTerm(i0, j0, k0, d.gg[1], 1.0f - u, u, -1.0f, 1.0f, 1.0f - w, w);
-        if (d.gg[2] != 0.0f) cellTerm(i0, j0, k0, d.gg[2], 1.0f - u, u, 1.0f - v, v, -1.0f, 1.0f);
-    }
-    if (d.gn != 0.0f) singleTerm(int32_t(rintf(p[0])), int32_t(rintf(p[1])), int32_t(rintf(p[2])), d.gn);
-    auto corners = [&](int t) { return T[t].single ? 1 : 8; };
-    for (int t = 0; t < nt; ++t) {
-        for (int c = 0; c < corners(t); ++c) {
-            const int32_t X = T[t].o[0] + (c >> 2), Y = T[t].o[1] + ((c >> 1) & 1), Z = T[t].o[2] + (c & 1);
-            bool seen = false;
-            for (int t2 = 0; t2 < t && !seen; ++t2)
-                for (int c2 = 0; c2 < corners(t2); ++c2)
-                    if (T[t2].o[0] + (c2 >> 2) == X && T[t2].o[1] + ((c2 >> 1) & 1) == Y && T[t2].o[2] + (c2 & 1) == Z) {
-                        seen = true;
-                        break;
-                    }
-            if (seen) continue;
-            float sum = 0.0f;
-            for (int t2 = t; t2 < nt; ++t2)
-                for (int c2 = 0; c2 < corners(t2); ++c2)
-                    if (T[t2].o[0] + (c2 >> 2) == X && T[t2].o[1] + ((c2 >> 1) & 1) == Y && T[t2].o[2] + (c2 & 1) == Z)
-                        sum += T[t2].single ? T[t2].s
-                                            : ((T[t2].s * T[t2].A[c2 >> 2]) * T[t2].B[(c2 >> 1) & 1]) * T[t2].C[c2 & 1];
-            emit(X, Y, Z, sum);
-        }
-    }
-}
-
-// True when every voxel the query's terms reach lies in the plus-shaped block around its cell
-// (cell + [-1, 2] on one axis, cell + [0, 1] on the others): always, except for FD6 sample points
-// whose p +- 1 rounds into a cell other than the neighbouring one.
-__host__ __device__ __forceinline__ bool adjointInBlock(const float p[3], int mode)
-{
-    if (mode != 1) return true;
+    if (d.gv != 0.0f) cellTerm(i0, j0, k0, d.gv, 1.0f - u, u, 1.0f - v, v, 1.0f - t, t);
     float q[6][3];
     fd6Points(p, q);
-    bool ok = true;
+    const float fd[3] = {k.fdx, k.fdy, k.fdz};
 #pragma unroll
-    for (int t = 0; t < 6; ++t) {
-        const int ax = t >> 1;
-        const float expect = floorf(p[ax]) + ((t & 1) ? -1.0f : 1.0f);
-        ok = ok && floorf(q[t][ax]) == expect;
+    for (int n = 0; n < 6; ++n) {
+        const float s0 = d.gg[n >> 1] * fd[n >> 1];
+        const float s = (n & 1) ? -s0 : s0;
+        if (s == 0.0f) continue;
+        const float gx = floorf(q[n][0]), gy = floorf(q[n][1]), gz = floorf(q[n][2]);
+        const float a = q[n][0] - gx, b = q[n][1] - gy, e = q[n][2] - gz;
+        cellTerm(int32_t(gx), int32_t(gy), int32_t(gz), s, 1.0f - a, a, 1.0f - b, b, 1.0f - e, e);
     }
-    return ok;
+    if (d.gn != 0.0f && terms == mine && c == 0) {
+        x = int32_t(rintf(p[0]));
+        y = int32_t(rintf(p[1]));
+        z = int32_t(rintf(p[2]));
+        w = d.gn;
+        have = true;
+    }
+    float sum = 0.0f;
+    bool first = have;
+#pragma unroll 4
+    for (int j = 0; j < 64; ++j) {
+        const bool same = __builtin_amdgcn_readlane(int(have), j) && __builtin_amdgcn_readlane(x, j) == x &&
+                          __builtin_amdgcn_readlane(y, j) == y && __builtin_amdgcn_readlane(z, j) == z;
+        const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+        if (same) {
+            first = first && j >= int(lane);
+            sum += wj;
+        }
+    }
+    if (first) emit(x, y, z, sum);
 }
 
 // Block form of the same sums (requires adjointInBlock): 32 register accumulators at constant
@@ -381,20 +634,53 @@ __device__ __forceinline__ int64_t adjointKey(const GridView& g, const Probe& pr
     else return pr.leaf ? int64_t((uint64_t(pr.leaf - g.leaf0) >> 5) / 67u) * 512 + pr.n : -1;
 }
 
-// One query's adjoint through the lane accessor, added into accum with int64 atomics.
+// One query per lane, added into accum with int64 atomics; every lane of the wavefront calls this,
+// `valid` or not.
 template<uint32_t GT>
-__device__ __forceinline__ void sampleAdjointOne(Accessor<GT>& acc, const GridView& g, const float p[3],
-                                                 const SampleGrad& d, int mode, const SampleConsts& k, float scale,
-                                                 unsigned long long* __restrict__ accum, bool& ok)
+__device__ __forceinline__ void sampleAdjointLanes(const GridView& g, bool valid, const float p[3], const SampleGrad& d,
+                                                   int mode, const SampleConsts& k, float scale,
+                                                   unsigned long long* __restrict__ accum, bool& ok)
 {
     auto emit = [&](int32_t x, int32_t y, int32_t z, float sum) {
         const long long q = toFixedSat(sum * scale, ok);
         if (q == 0) return;
+        Accessor<GT> acc(g);
         const int64_t key = adjointKey<GT>(g, acc.probe(x, y, z));
         if (key >= 0) atomicAdd(accum + key, static_cast<unsigned long long>(q));
     };
-    if (adjointInBlock(p, mode)) sampleAdjointBlock(p, d, mode, k, emit);
-    else sampleAdjointGeneral(p, d, mode, k, emit);
+    const bool off = valid && !adjointInBlock(p, mode);
+    if (valid && !off) {
+        BlockSlots B;
+        if (resolveBlock<GT>(g, int32_t(floorf(p[0])), int32_t(floorf(p[1])), int32_t(floorf(p[2])), true, B)) {
+            auto staged = [&](int32_t x, int32_t y, int32_t z, float sum) {
+                const long long q = toFixedSat(sum * scale, ok);
+                if (q == 0) return;
+                const uint32_t leaf = pickSlot(B, B.leaf, x, y, z), n = Accessor<GT>::leafOffset(x, y, z);
+                int64_t key;
+                if constexpr (GT == GT_ONINDEX)
+                    key = leaf != kNoLeaf ? int64_t(Codec<GT_ONINDEX>::index(g.leaf0 + (uint64_t(leaf) << 5), n))
+                                          : int64_t(pickSlot(B, B.index, x, y, z));
+                else
+                    key = leaf != kNoLeaf ? int64_t(leaf / 67u) * 512 + n : -1;
+                if (key >= 0) atomicAdd(accum + key, static_cast<unsigned long long>(q));
+            };
+            sampleAdjointBlock(p, d, mode, k, staged);
+        } else {
+            sampleAdjointBlock(p, d, mode, k, emit);
+        }
+    }
+    uint64_t todo = __ballot(off);
+    while (todo) {
+        const int src = __builtin_ctzll(todo);
+        todo &= todo - 1u;
+        const float P[3] = {__shfl(p[0], src, 64), __shfl(p[1], src, 64), __shfl(p[2], src, 64)};
+        SampleGrad D;
+        D.gn = __shfl(d.gn, src, 64);
+        D.gv = __shfl(d.gv, src, 64);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) D.gg[a] = __shfl(d.gg[a], src, 64);
+        sampleAdjointWave(P, D, mode, k, emit);
+    }
 }
 
 inline SampleConsts sampleConsts(const GridView& g)

@@ -1,0 +1,69 @@
+"""Point queries below the binned threshold (staged lookups of the block around a query) and their
+adjoint against the oracle, bit for bit: points on slot, node and root-tile boundaries, FD6 samples that
+round into a farther cell, far outside the grid and at the ends of the integer range, and batches that
+end inside a wavefront.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def grids():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import openvdb_amd as nvq
+    torus = nvq.tools.create_level_set_torus(50.0, 14.0, (0.0, 0.0, 0.0), 1.0, 3.0)  # eight root tiles
+    fog = nvq.tools.create_fog_fbm([4070, -30, 100, 4133, 33, 163], seed=5, amplitude=8.0)  # active tiles
+    out = {"torus": torus, "fog": fog}
+    for c in ("fp4", "fp8", "fp16", "fpn"):
+        out["torus_" + c] = nvq.tools.quantize(torus, c, 1e-3)
+    return nvq, out
+
+
+def _points(d, n):
+    r = np.random.default_rng(n)
+    lo, hi = np.array(d.index_bbox[:3], np.float64), np.array(d.index_bbox[3:], np.float64) + 1
+    p = (r.random((n, 3)) * (hi - lo + 20) + lo - 10).astype(np.float32)
+    k = n // 8
+    p[:k] = np.rint(p[:k] / 8) * 8 + r.integers(-2, 3, (k, 3))                   # around slot boundaries
+    p[k:2 * k] = np.nextafter(np.rint(p[k:2 * k]), np.float32(0))                # p +- 1 rounds up a cell
+    p[2 * k:3 * k] = r.choice([-4096.0, 0.0, 4096.0, 128.0], (k, 3)) + r.normal(0, 1.5, (k, 3))
+    if n > 60:
+        p[-1] = 1e9
+        p[-2] = [-2.1e9, 0.5, 3.0]
+        p[-3] = [16777216.0, 1.0, 1.0]
+    return p
+
+
+@pytest.mark.parametrize("name", ["torus", "fog", "torus_fp4", "torus_fp8", "torus_fp16", "torus_fpn"])
+@pytest.mark.parametrize("n", [1, 65, 20011])
+def test_staged_queries(oracle, grids, name, n):
+    nvq, hosts = grids
+    host = hosts[name]
+    d = nvq.DeviceGrid(host)
+    p = _points(d, n)
+    for mode in (1, 2, 3):
+        got = nvq.ops.sample(d, torch.from_numpy(p).cuda(), grad_mode=mode)
+        for a, b in zip(got, oracle.sample(host, p, grad_mode=mode)):
+            assert np.array_equal(a.cpu().numpy().view(np.uint32), np.ascontiguousarray(b).view(np.uint32)), mode
+
+
+@pytest.mark.parametrize("n", [1, 65, 5003])
+def test_staged_adjoint(oracle, grids, n):
+    nvq, hosts = grids
+    for name in ("torus", "fog"):
+        d = nvq.DeviceGrid(hosts[name])
+        p = _points(d, n)
+        r = np.random.default_rng(7)
+        gn, gv, gg = (r.normal(size=s).astype(np.float32) for s in ((n,), (n,), (n, 3)))
+        gv[::3] = 0.0
+        gg[::5] = 0.0
+        x = torch.from_numpy(p).cuda()
+        for mode in (1, 2, 3):
+            acc = nvq.ops.sample_backward(d, x, *(torch.from_numpy(a).cuda() for a in (gn, gv, gg)), mode)
+            want, over = oracle.sample_bwd_fixed(hosts[name], p, gn, gv, gg, mode, shift=40)
+            assert not over
+            assert np.array_equal(acc.cpu().numpy(), np.asarray(want).reshape(-1)), (name, mode)
