@@ -354,8 +354,9 @@ struct MultiArgs {
     uint32_t k;
     uint32_t totalTiles;
 };
-int multiQuery(const MultiArgs& A, const float* eye, const float* dir, float dt, float sigma, uint8_t* hit,
-               int32_t* ijk, float* a, float* b, float* normal, hipStream_t s);
+// views[j]: the host copy of grid j's view.
+int multiQuery(const MultiArgs& A, const GridView* const* views, const float* eye, const float* dir, float dt, float sigma,
+               uint8_t* hit, int32_t* ijk, float* a, float* b, float* normal, hipStream_t s);
 // The same with the queue counters in the library's per-device array: no allocation.
 int multiQueryNoAlloc(const MultiArgs& A, const float* eye, const float* dir, float dt, float sigma, uint8_t* hit,
                       int32_t* ijk, float* a, float* b, float* normal, hipStream_t s);

@@ -932,7 +932,9 @@ int nvq_multi_query(const nvq_grid* const* host_grids, uint32_t k, const uint64_
     MultiArgs A;
     const int st = makeMultiArgs(host_grids, k, host_ray_offsets, host_image_width, host_ops, eye, dir, dt, A);
     if (st != NVQ_OK || A.totalTiles == 0) return st;
-    return multiQuery(A, eye, dir, dt, sigma_t, hit, ijk, out_a, out_b, normal, S(stream)) == 0 ? NVQ_OK : NVQ_ERR_HIP;
+    const GridView* views[kMaxGrids];
+    for (uint32_t j = 0; j < k; ++j) views[j] = &host_grids[j]->view;
+    return multiQuery(A, views, eye, dir, dt, sigma_t, hit, ijk, out_a, out_b, normal, S(stream)) == 0 ? NVQ_OK : NVQ_ERR_HIP;
 }
 
 int nvq_multi_query_noalloc(const nvq_grid* const* host_grids, uint32_t k, const uint64_t* host_ray_offsets,

@@ -291,6 +291,16 @@ __device__ __forceinline__ bool isoCrossingSlots(const SlotMap& M, const GridVie
 // the table's 32-bit offsets.  launchSlotMap builds it in `mem` (256-byte aligned).
 // `parts`: kMapBricks, kMapSigns (against `iso`).
 size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts);
+// One map of a multi-grid call: the grid's view on the host and on the device, and the memory its map
+// is built in (nullptr: none, and maps[j].entry is null).
+struct MapJob {
+    const GridView* host;
+    const GridView* device;
+    char* mem;
+    uint32_t parts;
+};
+// Builds the maps of `n` grids (iso 0) with a few launches and stores them in maps[n], device memory.
+int launchSlotMaps(const MapJob* jobs, uint32_t n, SlotMap* maps, hipStream_t s);
 int launchSlotMap(const GridView& g, char* mem, SlotMap& M, uint32_t parts, float iso, hipStream_t s);
 
 } // namespace nvq

@@ -179,3 +179,25 @@ def test_adjoint_over_blocks(oracle, name, w, h):
 def _leaf_bytes(host):
     off, count = 672 + int(np.frombuffer(host, np.int64, 1, 672)[0]), int(np.frombuffer(host, np.uint32, 1, 704)[0])
     return slice(off, off + 2144 * count)
+
+
+@pytest.mark.parametrize("codec", ["float", "fp8", "fpn"])
+def test_multi_query_over_maps_equals_the_accessor_launch(codec):
+    """nvq_multi_query (slot maps, tiles left open answered again) against nvq_multi_query_noalloc."""
+    nvq = _nvq()
+    hosts = [_level_set(nvq, "sphere"), _host(nvq, "fog"), _level_set(nvq, "torus"), _host(nvq, "tiles")]
+    if codec != "float":
+        hosts = [nvq.tools.quantize(h, codec, 1e-3) for h in hosts]
+    else:
+        hosts += [_flagged(hosts[0]), _flagged(hosts[1])]
+    grids = [nvq.DeviceGrid(h) for h in hosts]
+    for w, h in ((9, 7), (203, 121)):  # below and above the tile count that is ordered
+        rays = [_image(d, w, h) for d in grids]
+        eye, dirs = (torch.cat(x) for x in zip(*rays))
+        offs = [w * h * j for j in range(len(grids) + 1)]
+        for widths in ([w] * len(grids), [0] + [w] * (len(grids) - 1)):
+            a = nvq.ops.multi_query(grids, eye, dirs, offs, widths, 0.5, 0.05)
+            b = nvq.ops.multi_query(grids, eye, dirs, offs, widths, 0.5, 0.05, noalloc=True)
+            for x, y in zip(a, b):
+                assert torch.equal(x.view(torch.uint8), y.view(torch.uint8))
+        assert int(a[0].sum()) > 0 and float(a[2].max()) > 0.0
