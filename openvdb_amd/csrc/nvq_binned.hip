@@ -14,7 +14,7 @@
 //   radix sort     : (key, point) pairs of the marked queries (rocPRIM/hipCUB DeviceRadixSort)
 //   k_bin_bounds   : [begin, end) of every non-empty bin in the sorted order
 //   k_bin_sample   : one 512-thread workgroup per bin stages the 20^3 brick of voxel values around the bin in
-//                    LDS (ReadAccessor::getValue semantics, so results are bit-identical) and
+//                    LDS, a row of eight voxels per load (ReadAccessor::getValue semantics, so results are bit-identical) and
 //                    evaluates the bin's queries from it; each query's results go to its original
 //                    index as one 64-byte record, written by the four lanes of a quad
 //   k_sample_list  : queries whose stencil leaves the brick run through the lane accessor
@@ -27,6 +27,7 @@
 #include "nvq_internal.h"
 #include "nvq_profile.h"
 #include "nvq_sample.h"
+#include "nvq_slots.h"
 
 #include <hip/hip_runtime.h>
 
@@ -474,7 +475,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample(GridView g, BinLayou
                                                          SampleConsts k, uint32_t* __restrict__ spill,
                                                          uint32_t* __restrict__ spillCount)
 {
-    __shared__ float brick[kBrickVox];
+    __shared__ __align__(16) float brick[kBrickVox];
     __shared__ const uint8_t* slotLeaf[64]; // leaf node of each 8^3 slot the brick overlaps, or null
     __shared__ float slotValue[64];         // the slot's tile or background value when it has no leaf
     const uint32_t b = blockIdx.x;
@@ -484,28 +485,36 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample(GridView g, BinLayou
                    bx = b / (uint32_t(L.nb[2]) * uint32_t(L.nb[1]));
     const int32_t o[3] = {L.lo[0] + (int32_t(bx) << kBinLog2) - 1, L.lo[1] + (int32_t(by) << kBinLog2) - 1,
                           L.lo[2] + (int32_t(bz) << kBinLog2) - 1};
-    // The brick overlaps at most 4x4x4 aligned 8^3 slots; inside one slot every voxel is read from
-    // one leaf or, without a leaf, equals one tile or background value.  One tree walk per slot
-    // (64 lanes in parallel), then every brick voxel is an independent load (ReadAccessor::getValue
-    // semantics, NanoVDB.h:5370-5377).
+    // The brick starts on a slot boundary and overlaps 3x3x3 aligned 8^3 slots; inside one slot every
+    // voxel is read from one leaf or, without a leaf, equals one tile or background value.  One tree
+    // walk per slot (27 lanes in parallel), then the rows of eight voxels are independent wide loads
+    // (ReadAccessor::getValue semantics, NanoVDB.h:5370-5377).
     const int32_t s0[3] = {o[0] >> 3, o[1] >> 3, o[2] >> 3};
-    const int32_t ns[3] = {((o[0] + kBrick - 1) >> 3) - s0[0] + 1, ((o[1] + kBrick - 1) >> 3) - s0[1] + 1,
-                           ((o[2] + kBrick - 1) >> 3) - s0[2] + 1};
-    if (threadIdx.x < uint32_t(ns[0] * ns[1] * ns[2])) {
+    if (threadIdx.x < 27u) {
         const int32_t t = int32_t(threadIdx.x);
-        const int32_t sx = t / (ns[1] * ns[2]), sy = (t / ns[2]) % ns[1], sz = t % ns[2];
+        const int32_t sx = t / 9, sy = (t / 3) % 3, sz = t % 3;
         Accessor<GT> acc(g);
         const Probe pr = acc.probe((s0[0] + sx) << 3, (s0[1] + sy) << 3, (s0[2] + sz) << 3);
         slotLeaf[(sx * 4 + sy) * 4 + sz] = pr.leaf;
         slotValue[(sx * 4 + sy) * 4 + sz] = pr.value;
     }
     __syncthreads();
-    for (int v = threadIdx.x; v < kBrickVox; v += kBinThreads) {
-        const int32_t x = v / (kBrick * kBrick), y = (v / kBrick) % kBrick, z = v % kBrick;
-        const int32_t gx = o[0] + x, gy = o[1] + y, gz = o[2] + z;
-        const int slot = (((gx >> 3) - s0[0]) * 4 + ((gy >> 3) - s0[1])) * 4 + ((gz >> 3) - s0[2]);
+    // row (x, y) of the brick in slot layer zs: voxels 8 zs .. 8 zs + 7 (the last layer: + 3)
+    for (uint32_t r = threadIdx.x; r < uint32_t(kBrick * kBrick) * 4u; r += kBinThreads) {
+        const uint32_t zs = r & 3u, row = r >> 2, x = row / uint32_t(kBrick), y = row % uint32_t(kBrick);
+        if (zs == 3u) continue;
+        const uint32_t slot = ((x >> 3) * 4u + (y >> 3)) * 4u + zs;
         const uint8_t* leaf = slotLeaf[slot];
-        brick[v] = leaf ? Codec<GT>::get(leaf, Accessor<GT>::leafOffset(gx, gy, gz), g.channel) : slotValue[slot];
+        float v[8];
+        if (leaf) {
+            leafRow<GT>(leaf, (x & 7u) * 8u + (y & 7u), g.channel, v);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = slotValue[slot];
+        }
+        float4* out = reinterpret_cast<float4*>(brick + row * uint32_t(kBrick) + 8u * zs);
+        out[0] = make_float4(v[0], v[1], v[2], v[3]);
+        if (zs < 2u) out[1] = make_float4(v[4], v[5], v[6], v[7]);
     }
     __syncthreads();
     // wave-uniform loop (the record store is a wave-wide operation): 64 consecutive queries per wave;
@@ -521,52 +530,20 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample(GridView g, BinLayou
         const float p[3] = {t.x, t.y, t.z};
         const float fx = floorf(p[0]), fy = floorf(p[1]), fz = floorf(p[2]);
         const int32_t ci = int32_t(fx) - o[0], cj = int32_t(fy) - o[1], ck = int32_t(fz) - o[2];
-        // every FD6 sample cell lies in [cell-1, cell+2] (p +- 1 rounds at most one voxel further up),
-        // so the whole stencil is inside the brick iff the cell is in [1, kBrick-4]
+        // the block [cell-1, cell+2]^3 lies in the brick iff the cell is in [1, kBrick-4]; FD6 samples that
+        // round out of the block go to the list too
         if (valid && (uint32_t(ci - 1) > uint32_t(kBrick - 5) || uint32_t(cj - 1) > uint32_t(kBrick - 5) ||
-                      uint32_t(ck - 1) > uint32_t(kBrick - 5))) {
+                      uint32_t(ck - 1) > uint32_t(kBrick - 5) || !adjointInBlock(p, mode))) {
             spill[atomicAdd(spillCount, 1u)] = id;
             valid = false;
         }
-        float nnv = 0.0f, vv = 0.0f;
-        float g3[3] = {0.0f, 0.0f, 0.0f};
+        SampleOut out{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
         if (valid) {
-            auto load = [&](int32_t cb, Cell& c) {
-#pragma unroll
-                for (int a = 0; a < 2; ++a)
-#pragma unroll
-                    for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-                        for (int e = 0; e < 2; ++e) c.v[a][bb][e] = brick[cb + (a * kBrick + bb) * kBrick + e];
-            };
-            auto cell = [&](float qx, float qy, float qz) -> float {
-                const float gx = floorf(qx), gy = floorf(qy), gz = floorf(qz);
-                const int32_t cb = ((int32_t(gx) - o[0]) * kBrick + (int32_t(gy) - o[1])) * kBrick + (int32_t(gz) - o[2]);
-                Cell c;
-                load(cb, c);
-                return trilerp(c, qx - gx, qy - gy, qz - gz);
-            };
-            const int32_t c0 = (ci * kBrick + cj) * kBrick + ck;
-            if (wantNN) {
-                const int32_t ri = int32_t(rintf(p[0])) - o[0], rj = int32_t(rintf(p[1])) - o[1], rk = int32_t(rintf(p[2])) - o[2];
-                nnv = brick[(ri * kBrick + rj) * kBrick + rk];
-            }
-            if (wantVal) vv = cell(p[0], p[1], p[2]);
-            if (mode == 1) {
-                g3[0] = (cell(p[0] + 1.0f, p[1] + 0.0f, p[2] + 0.0f) - cell(p[0] - 1.0f, p[1] - 0.0f, p[2] - 0.0f)) * k.fdx;
-                g3[1] = (cell(p[0] + 0.0f, p[1] + 1.0f, p[2] + 0.0f) - cell(p[0] - 0.0f, p[1] - 1.0f, p[2] - 0.0f)) * k.fdy;
-                g3[2] = (cell(p[0] + 0.0f, p[1] + 0.0f, p[2] + 1.0f) - cell(p[0] - 0.0f, p[1] - 0.0f, p[2] - 1.0f)) * k.fdz;
-            } else if (mode == 2) {
-                g3[0] = k.gsInv2dx * (brick[c0 + kBrick * kBrick] - brick[c0 - kBrick * kBrick]);
-                g3[1] = k.gsInv2dx * (brick[c0 + kBrick] - brick[c0 - kBrick]);
-                g3[2] = k.gsInv2dx * (brick[c0 + 1] - brick[c0 - 1]);
-            } else if (mode == 3) {
-                Cell C;
-                load(c0, C);
-                trilinearGradient(C, p[0] - fx, p[1] - fy, p[2] - fz, g3);
-            }
+            const float* c0 = brick + (ci * kBrick + cj) * kBrick + ck;
+            out = sampleFromBlock([&](int x, int y, int z) { return c0[(x * kBrick + y) * kBrick + z]; }, p, wantNN, wantVal,
+                                  mode, k);
         }
-        storeRecQuad(rec, valid, id, nnv, vv, g3);
+        storeRecQuad(rec, valid, id, out.nn, out.val, out.g);
     }
 }
 
@@ -849,7 +826,8 @@ bool makeLayout(const GridView& g, BinLayout& L)
     for (int a = 0; a < 3; ++a) {
         // whole leaves and two voxels more: points in a leaf that reaches past the bbox of the active voxels
         // would otherwise leave their brick and go through the lane kernel one by one
-        const int64_t lo = (int64_t(g.bbox[a]) & ~int64_t(7)) - 2, hi = (int64_t(g.bbox[3 + a]) | 7) + 2;
+        // and a brick starts with a leaf: it overlaps three slots per axis instead of four
+        const int64_t lo = (int64_t(g.bbox[a]) & ~int64_t(7)) - 7, hi = (int64_t(g.bbox[3 + a]) | 7) + 2;
         const int64_t nb = ((hi - lo) >> kBinLog2) + 1;
         if (nb > (int64_t(1) << 20)) return false;
         L.lo[a] = int32_t(lo);

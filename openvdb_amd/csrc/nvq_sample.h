@@ -309,17 +309,16 @@ __device__ __forceinline__ float blockVoxel(const GridView& g, const BlockSlots&
     return v;
 }
 
-// sampleEval over resolved slots, with its operations in its order, for queries whose FD6 cells are the
-// neighbouring ones (adjointInBlock).  False: through the accessor.
-template<uint32_t GT>
-__device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3], bool wantNN, bool wantVal, int mode,
-                                             const SampleConsts& k, SampleOut& r)
+// sampleEval with its operations in its order, from the voxels of the block around the query's cell:
+// at(dx, dy, dz) is the voxel at that offset from the cell's corner.  For queries whose FD6 cells are
+// the neighbouring ones (adjointInBlock) and whose nearest voxel is a corner of the cell.
+template<class At>
+__device__ __forceinline__ SampleOut sampleFromBlock(At&& at, const float p[3], bool wantNN, bool wantVal, int mode,
+                                                     const SampleConsts& k)
 {
     const float fx = floorf(p[0]), fy = floorf(p[1]), fz = floorf(p[2]);
-    const int32_t i0 = int32_t(fx), j0 = int32_t(fy), k0 = int32_t(fz);
-    const int32_t ri = int32_t(rintf(p[0])) - i0, rj = int32_t(rintf(p[1])) - j0, rk = int32_t(rintf(p[2])) - k0;
-    BlockSlots B;
-    if (((ri | rj | rk) & ~1) || !resolveBlock<GT>(g, i0, j0, k0, false, B)) return false;
+    const int32_t ri = int32_t(rintf(p[0])) - int32_t(fx), rj = int32_t(rintf(p[1])) - int32_t(fy),
+                  rk = int32_t(rintf(p[2])) - int32_t(fz);
     const float u = p[0] - fx, v = p[1] - fy, w = p[2] - fz;
     Cell C;
 #pragma unroll
@@ -327,8 +326,8 @@ __device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3]
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
-            for (int e = 0; e < 2; ++e) C.v[a][b][e] = blockVoxel<GT>(g, B, i0 + a, j0 + b, k0 + e);
-    r = SampleOut{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
+            for (int e = 0; e < 2; ++e) C.v[a][b][e] = at(a, b, e);
+    SampleOut r{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
     if (mode == 1) {
         // the layers next to the cell: [axis][side][the other two axes]
         float L[3][2][2][2];
@@ -338,9 +337,9 @@ __device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3]
             for (int a = 0; a < 2; ++a)
 #pragma unroll
                 for (int b = 0; b < 2; ++b) {
-                    L[0][s][a][b] = blockVoxel<GT>(g, B, i0 + (s ? 2 : -1), j0 + a, k0 + b);
-                    L[1][s][a][b] = blockVoxel<GT>(g, B, i0 + a, j0 + (s ? 2 : -1), k0 + b);
-                    L[2][s][a][b] = blockVoxel<GT>(g, B, i0 + a, j0 + b, k0 + (s ? 2 : -1));
+                    L[0][s][a][b] = at(s ? 2 : -1, a, b);
+                    L[1][s][a][b] = at(a, s ? 2 : -1, b);
+                    L[2][s][a][b] = at(a, b, s ? 2 : -1);
                 }
         if (wantNN) r.nn = pick(C, ri, rj, rk);
         if (wantVal) r.val = trilerp(C, u, v, w);
@@ -370,19 +369,33 @@ __device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3]
         r.g[0] = (f[0][1] - f[0][0]) * k.fdx;
         r.g[1] = (f[1][1] - f[1][0]) * k.fdy;
         r.g[2] = (f[2][1] - f[2][0]) * k.fdz;
-        return true;
+        return r;
     }
     if (wantNN) r.nn = pick(C, ri, rj, rk);
     if (wantVal) r.val = trilerp(C, u, v, w);
     if (mode == 2) {
-        const float mx = blockVoxel<GT>(g, B, i0 - 1, j0, k0), my = blockVoxel<GT>(g, B, i0, j0 - 1, k0),
-                    mz = blockVoxel<GT>(g, B, i0, j0, k0 - 1);
+        const float mx = at(-1, 0, 0), my = at(0, -1, 0),
+                    mz = at(0, 0, -1);
         r.g[0] = k.gsInv2dx * (C.v[1][0][0] - mx);
         r.g[1] = k.gsInv2dx * (C.v[0][1][0] - my);
         r.g[2] = k.gsInv2dx * (C.v[0][0][1] - mz);
     } else if (mode == 3) {
         trilinearGradient(C, u, v, w, r.g);
     }
+    return r;
+}
+
+// Over resolved slots, for queries adjointInBlock.  False: through the accessor.
+template<uint32_t GT>
+__device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3], bool wantNN, bool wantVal, int mode,
+                                             const SampleConsts& k, SampleOut& r)
+{
+    const int32_t i0 = int32_t(floorf(p[0])), j0 = int32_t(floorf(p[1])), k0 = int32_t(floorf(p[2]));
+    const int32_t ri = int32_t(rintf(p[0])) - i0, rj = int32_t(rintf(p[1])) - j0, rk = int32_t(rintf(p[2])) - k0;
+    BlockSlots B;
+    if (((ri | rj | rk) & ~1) || !resolveBlock<GT>(g, i0, j0, k0, false, B)) return false;
+    r = sampleFromBlock([&](int x, int y, int z) { return blockVoxel<GT>(g, B, i0 + x, j0 + y, k0 + z); }, p, wantNN,
+                        wantVal, mode, k);
     return true;
 }
 

@@ -78,6 +78,41 @@ __device__ __forceinline__ v2f loadPair(const float* p)
     return v;
 }
 
+// Decoded values of the eight voxels (x, y, 0..7) of a leaf, row = 8 x + y: one or two wide loads.
+template<uint32_t GT>
+__device__ __forceinline__ void leafRow(const uint8_t* leaf, uint32_t row, const float* channel, float v[8])
+{
+    if constexpr (GT == GT_FLOAT) {
+        const float4* p = reinterpret_cast<const float4*>(leaf + kLeafData + 32u * row);
+        const float4 a = p[0], b = p[1];
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else if constexpr (GT == GT_FP16 || GT == GT_FP8 || GT == GT_FP4) {
+        constexpr int kBits = GT == GT_FP16 ? 16 : (GT == GT_FP8 ? 8 : 4), kWords = kBits / 4;
+        uint32_t w[kWords];
+        __builtin_memcpy(w, leaf + kLeafData + row * uint32_t(kBits), sizeof(w));
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            v[k] = dequant(leaf, (w[k * kBits / 32] >> (k * kBits % 32)) & ((1u << kBits) - 1u));
+    } else if constexpr (GT == GT_ONINDEX) {
+        // the row is one byte of the value mask: its active voxels have consecutive indices
+        const uint32_t w = row >> 3, shift = 8u * (row & 7u);
+        const uint64_t word = ld_u64(leaf + kLeafVMask + 8u * w);
+        uint64_t at = ld_u64(leaf + kIdxLeafOffset) + uint64_t(__popcll(word & ((uint64_t(1) << shift) - 1u)));
+        if (w) at += (ld_u64(leaf + kIdxLeafPrefix) >> (9u * (w - 1u))) & 511u;
+        const uint32_t bits = uint32_t(word >> shift) & 255u;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const bool on = (bits >> k) & 1u;
+            v[k] = channel[on ? at : 0u];
+            at += on ? 1u : 0u;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = Codec<GT>::get(leaf, 8u * row + k, channel);
+    }
+}
+
 // Corners of the cell at brick offset `at` (brick * kBrickFloats + (x * 9 + y) * 9 + z)
 __device__ __forceinline__ void brickCell(const SlotMap& M, uint32_t at, Cell& c)
 {
