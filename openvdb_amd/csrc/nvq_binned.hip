@@ -895,6 +895,10 @@ void launchClassify(const GridView& g, const Bins& B, const SlotTable& T, float*
     ProfScope prof("k_bin_classify", s);
     const uint64_t words = (count + 31) / 32;
     const uint32_t ldsWords = words <= kLdsLeafWords ? uint32_t(words) : 0u;
+    // A large bitmap is staged by no more workgroups than the CUs' LDS holds at once: the 41 KB of a 512^3
+    // fog took 198 us with 4096 workgroups (168 MB staged in all) and 160 us with 768; the 26 KB of
+    // the torus 343 us with 4096 and 355 with 1536, so smaller ones keep the workgroups
+    if (ldsWords > 8192u) blocks = std::min<uint32_t>(blocks, 256u * ((160u << 10) / (ldsWords * 4u + 64u)));
     hipLaunchKernelGGL(k_bin_classify, dim3(blocks), dim3(kThreads), size_t(ldsWords) * 4u, s, g, T, xyz, B.n, B.chunks,
                        world, c.mode, ldsWords, B.cflags, B.counts);
 }

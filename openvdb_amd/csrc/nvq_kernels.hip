@@ -103,6 +103,41 @@ __global__ __launch_bounds__(kBlock) void k_get_value(GridView g, const int32_t*
     }
 }
 
+// The same over a slot table: two lookups (slot, leaf) instead of the walk's five.  Voxels outside the
+// table, or in a slot it leaves open, go through the tree.  Bound by the L1's and L2's line rate: 10.6 M
+// shuffled voxels of an index grid 443 -> 370 us (two or four voxels per lane at a time: the same).
+constexpr uint64_t kValueMapMin = 1u << 18;
+template<uint32_t GT>
+__global__ __launch_bounds__(kBlock) void k_get_value_slots(SlotMap M, GridView g, const int32_t* __restrict__ ijk,
+                                                            uint64_t n, float* __restrict__ val,
+                                                            uint8_t* __restrict__ active, uint32_t* __restrict__ dim)
+{
+    const uint64_t stride = uint64_t(gridDim.x) * kBlock;
+    for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += stride) {
+        const int32_t x = ijk[3 * i], y = ijk[3 * i + 1], z = ijk[3 * i + 2];
+        uint32_t slot, e = kSlotOther;
+        if (slotAt(M, x, y, z, slot)) e = M.entry[slot];
+        Probe p;
+        if (!(e & kSlotTile)) {
+            const uint8_t* leaf = slotLeaf(M, g, e);
+            const uint32_t v = Accessor<GT>::leafOffset(x, y, z);
+            p.value = Codec<GT>::get(leaf, v, g.channel);
+            p.active = maskOn(leaf + kLeafVMask, v);
+            p.dim = 1u;
+        } else if (e != kSlotOther) {
+            p.value = M.value[slot];
+            p.active = (e & kSlotTileOn) != 0;
+            p.dim = uint32_t(slotDim(e));
+        } else {
+            Accessor<GT> acc(g);
+            p = acc.probe(x, y, z);
+        }
+        if (val) val[i] = p.value;
+        if (active) active[i] = p.active ? 1 : 0;
+        if (dim) dim[i] = p.dim;
+    }
+}
+
 // ------------------------------------------------------------------ point sampling
 // 171 VGPRs uncapped (2 wavefronts per SIMD); at 4 (128, a 124-byte spill) 300,007 queries take 58.8 us
 // instead of 64.2, 1000 take 12.4 instead of 12.1.  Bound by the L1's line rate for the larger, by the
@@ -281,9 +316,13 @@ uint32_t gridStrideBlocks(uint64_t n)
 }
 
 template<uint32_t GT> struct RunGetValue {
-    static void run(const GridView& g, const int32_t* ijk, uint64_t n, float* val, uint8_t* act, uint32_t* dim, hipStream_t s)
+    static void run(const GridView& g, const SlotMap* M, const int32_t* ijk, uint64_t n, float* val, uint8_t* act,
+                    uint32_t* dim, hipStream_t s)
     {
-        hipLaunchKernelGGL(k_get_value<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, g, ijk, n, val, act, dim);
+        if (M)
+            hipLaunchKernelGGL(k_get_value_slots<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, *M, g, ijk, n, val, act, dim);
+        else
+            hipLaunchKernelGGL(k_get_value<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, g, ijk, n, val, act, dim);
     }
 };
 template<uint32_t GT> struct RunSample {
@@ -757,7 +796,14 @@ int nvq_get_value(const nvq_grid* grid, const int32_t* ijk, uint64_t n, float* v
 {
     if (!grid || !queryable(grid) || (n && !ijk)) return NVQ_ERR_INVALID_ARG;
     if (n == 0) return NVQ_OK;
-    return launchTyped<RunGetValue>(grid->view.type, grid->view, ijk, n, val, active, dim, S(stream));
+    // Large batches through a slot table: about 45 us per million slots to build, against about 7 us saved per
+    // million voxels, so from 8 voxels per slot on.
+    WorkspaceLease lease;
+    SlotMap M;
+    bool mapped = false;
+    if (n >= kValueMapMin && slotCount(grid->view) <= n / 8)
+        (void)acquireWithMap(lease, grid->view, n, 0u, 0.0f, 0, M, mapped, S(stream));
+    return launchTyped<RunGetValue>(grid->view.type, grid->view, mapped ? &M : nullptr, ijk, n, val, active, dim, S(stream));
 }
 
 int nvq_sample(const nvq_grid* grid, const float* xyz, uint64_t n, int world, float* nn, float* val, float* grad,

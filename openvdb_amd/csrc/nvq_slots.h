@@ -326,6 +326,7 @@ __device__ __forceinline__ bool isoCrossingSlots(const SlotMap& M, const GridVie
 // the table's 32-bit offsets.  launchSlotMap builds it in `mem` (256-byte aligned).
 // `parts`: kMapBricks, kMapSigns (against `iso`).
 size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts);
+uint64_t slotCount(const GridView& g); // ~0 where there is no table
 // One map of a multi-grid call: the grid's view on the host and on the device, and the memory its map
 // is built in (nullptr: none, and maps[j].entry is null).
 struct MapJob {

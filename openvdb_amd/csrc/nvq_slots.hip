@@ -285,6 +285,14 @@ bool layMap(const GridView& g, char* mem, uint32_t parts, SlotMap& M, MapMem& W)
 
 } // namespace
 
+uint64_t slotCount(const GridView& g)
+{
+    int32_t lo[3];
+    uint32_t n[3];
+    uint64_t count;
+    return slotBox(g, lo, n, count) ? count : ~uint64_t(0);
+}
+
 size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts)
 {
     int32_t lo[3];
