@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 
 // Over a slot map.  Rays that meet a slot the map leaves open start over through the accessor.
 // 128 VGPRs, 4 wavefronts per SIMD.  1024^2 rays through the 512^3 fog: 8.73 ms through the accessor,
-// 1.29 ms here and 0.16 ms for the map; 320x180 rays through a 128^3 index grid 2.50 -> 0.20 ms.
+// 1.29 ms here and 0.16 ms for the map.
 // Caps of 5 and 6 wavefronts (2 steps in flight, spills) were slower: 1.34 and 1.45 ms.
 template<uint32_t GT>
 __global__ __launch_bounds__(kBlock) void k_fog_march_slots(SlotMap M, GridView g, const GridView* whole, const float* __restrict__ eye,
@@ -273,6 +273,31 @@ __global__ __launch_bounds__(kBlock) void k_fog_march_slots(SlotMap M, GridView 
     uint64_t i;
     if (!scheduleOrdered(s, order, i)) return;
     if (!fogMarchSlots<kMarchBatch>(M, g, eye, dir, i, dt, sigma, Lout, Tout))
+        fogMarchRay<GT>(*whole, eye, dir, i, dt, sigma, Lout, Tout);
+}
+
+// Four lanes per ray (fogMarchQuad): a wavefront takes a quarter of a tile, 4x4 pixels or 16 rays.  Up to
+// kQuadTiles tiles, where the lanes that repeat a ray's walk would otherwise be missing from the chip.
+// Rays through the 512^3 fog, one lane and four per ray: 64^2 1302 and 912 us, 512^2 1602 and 965,
+// 800^2 1370 and 1103, 1024^2 1590 and 1561, 1200^2 1908 and 1997; through the 256^3 fog 640^2 527 and 359,
+// 1024^2 704 and 674, 1200^2 803 and 870.
+constexpr uint64_t kQuadTiles = 16384;
+template<uint32_t GT>
+__global__ __launch_bounds__(kBlock) void k_fog_march_quads(SlotMap M, GridView g, const GridView* whole,
+                                                            const float* __restrict__ eye, const float* __restrict__ dir,
+                                                            Sched s, const uint32_t* __restrict__ order, float dt,
+                                                            float sigma, float* __restrict__ Lout,
+                                                            float* __restrict__ Tout)
+{
+    const uint64_t wave = uint64_t(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+    if ((wave >> 2) >= s.tiles) return;
+    const uint64_t tile = order ? order[wave >> 2] : wave >> 2;
+    const uint32_t part = uint32_t(wave & 3u), r = (threadIdx.x & 63u) >> 2;
+    // ray r of the part as a lane of its tile
+    const uint32_t lane = s.width ? ((part >> 1) * 4u + (r >> 2)) * 8u + (part & 1u) * 4u + (r & 3u) : part * 16u + r;
+    uint64_t i;
+    if (!tileRay(s, tile, lane, i)) return; // whole quads
+    if (!fogMarchQuad(M, g, eye, dir, i, dt, sigma, Lout, Tout) && (threadIdx.x & 3u) == 0)
         fogMarchRay<GT>(*whole, eye, dir, i, dt, sigma, Lout, Tout);
 }
 
@@ -362,7 +387,10 @@ template<uint32_t GT> struct RunFogMarch {
                     const Sched& sc, const uint32_t* order, float dt, float sigma, float* L, float* T, hipStream_t s)
     {
         ProfScope prof("k_fog_march", s);
-        if (M)
+        if (M && sc.tiles <= kQuadTiles)
+            hipLaunchKernelGGL(k_fog_march_quads<GT>, dim3(uint32_t(sc.tiles)), dim3(kBlock), 0, s, *M, g, dg, eye, dir, sc,
+                               order, dt, sigma, L, T);
+        else if (M)
             hipLaunchKernelGGL(k_fog_march_slots<GT>, dim3(orderedBlocks(sc)), dim3(kBlock), 0, s, *M, g, dg, eye, dir,
                                sc, order, dt, sigma, L, T);
         else

@@ -122,9 +122,8 @@ __device__ __forceinline__ void fogMarchRay(const GridView& g, const float* __re
 // with nothing written, when the ray meets a slot the map does not resolve.
 //
 // Bound by the L1's line rate and the VALU in turn: per step four 8-byte loads that touch the
-// lines of 64 neighbouring cells, and about 60 instructions.  A batch of 4 hides the loads' latency
-// where few wavefronts are resident (57,600 rays: 0.24 ms at 2, 0.20 ms at 4) and costs nothing in a
-// full launch (1024^2 rays: 1.34 ms at 2, 1.29 ms at 4).
+// lines of 64 neighbouring cells, and about 60 instructions.  1024^2 rays: 1.34 ms with batches of 2,
+// 1.29 ms with 4.
 constexpr int kMarchBatch = 4;
 
 template<int B>
@@ -202,6 +201,101 @@ __device__ __forceinline__ bool fogMarchSlots(const SlotMap& M, const GridView& 
     }
     if (Lout) Lout[i] = L;
     if (Tout) Tout[i] = T;
+    return true;
+}
+
+// The same march by four lanes per ray: every lane of a quad walks the ray, lane q samples the q-th of
+// four steps, and all four composite them in order.  For launches too small to fill the chip, where
+// the time is that of one ray's chain of steps: a batch costs one sample and four compositings
+// instead of four of each.  `live`: the quad has a ray.
+__device__ __forceinline__ float quadLane(float x, int j)
+{
+    const int v = __float_as_int(x);
+    switch (j) {
+    case 0: return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x00, 0xf, 0xf, false));
+    case 1: return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0x55, 0xf, 0xf, false));
+    case 2: return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0xaa, 0xf, 0xf, false));
+    default: return __int_as_float(__builtin_amdgcn_mov_dpp(v, 0xff, 0xf, 0xf, false));
+    }
+}
+
+__device__ __forceinline__ bool fogMarchQuad(const SlotMap& M, const GridView& g, const float* __restrict__ eye,
+                                             const float* __restrict__ dir, uint64_t i, float dt, float sigma,
+                                             float* __restrict__ Lout, float* __restrict__ Tout)
+{
+    const uint32_t q = threadIdx.x & 3u;
+    const float e[3] = {eye[3 * i], eye[3 * i + 1], eye[3 * i + 2]};
+    const float d[3] = {dir[3 * i], dir[3 * i + 1], dir[3 * i + 2]};
+    float L = 0.0f, T = 1.0f;
+    Ray R = worldToIndexRay(g, e, d);
+    const float Eps = 0.000001f, Delta = 0.01f;
+    bool in = rayClip(R, g.bbox) && !(double(R.t1) > 1e20);
+    const float t0 = R.t0 + Eps, t1 = R.t1 - Eps;
+    in = in && !(t0 > t1);
+    if (in) {
+        float p[3];
+        rayAt(R, t0, p);
+        SlotCell c;
+        if (!slotCell(M, ifloor(p[0]), ifloor(p[1]), ifloor(p[2]), c)) return false;
+        HDDA h;
+        h.init(R, t0, t1, c.dim > 8 ? c.dim : 8);
+        for (;;) {
+            const float ta = h.t0;
+            const bool more = h.stepOnce();
+            const float tb = fminf(h.t0, t1);
+            const bool brick = !(c.entry & kSlotTile);
+            if ((brick || (c.entry & kSlotTileOn)) && ta < tb) {
+                const uint32_t base = brick ? c.entry * kBrickFloats : 0u;
+                float kf = ceilf(ta / dt);
+                while (kf * dt < tb) {
+                    // step numbers are whole floats: exact to 2^24, one at a time up there
+                    const bool whole = fabsf(kf) < 16777000.0f;
+                    const float t = (whole ? kf + float(q) : kf) * dt;
+                    const bool ok = (q == 0 || whole) && t < tb;
+                    const float x0 = __builtin_fmaf(t, R.dir[0], R.eye[0]), x1 = __builtin_fmaf(t, R.dir[1], R.eye[1]),
+                                x2 = __builtin_fmaf(t, R.dir[2], R.eye[2]);
+                    const float fx = floorf(x0), fy = floorf(x1), fz = floorf(x2);
+                    const uint32_t rx = uint32_t(int32_t(fx) - c.ox), ry = uint32_t(int32_t(fy) - c.oy),
+                                   rz = uint32_t(int32_t(fz) - c.oz);
+                    const bool fast = brick && (rx | ry | rz) < 8u;
+                    Cell cell;
+                    brickCell(M, fast ? base + (rx * 9u + ry) * 9u + rz : 0u, cell);
+                    float rho = trilerp(cell, x0 - fx, x1 - fy, x2 - fz);
+                    bool open = false;
+                    // a tile, or a position that rounding put just outside its slot
+                    if (ok && !fast) open = !slotTrilinear(M, x0, x1, x2, rho);
+                    const uint32_t quad = threadIdx.x & 60u;
+                    if ((__ballot(open) >> quad) & 15u) return false; // the whole quad
+                    const uint32_t valid = uint32_t(__ballot(ok) >> quad) & 15u;
+                    const float a = stepAbsorption(sigma, rho, dt);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float rj = quadLane(rho, j), aj = quadLane(a, j);
+                        const float Ln = L + T * (1.0f - aj) * rj, Tn = T * aj;
+                        const bool use = (valid >> j) & 1u;
+                        L = use ? Ln : L;
+                        T = use ? Tn : T;
+                    }
+                    if (!whole) {
+                        const float kn = kf + 1.0f;
+                        if (kn == kf) break;
+                        kf = kn;
+                    } else {
+                        if (valid != 15u) break;
+                        kf += 4.0f;
+                    }
+                }
+            }
+            if (!more) break;
+            rayAt(R, h.t0 + Delta, p);
+            if (!slotCell(M, ifloor(p[0]), ifloor(p[1]), ifloor(p[2]), c)) return false;
+            h.update(R, c.dim > 8 ? c.dim : 8);
+        }
+    }
+    if (q == 0) {
+        if (Lout) Lout[i] = L;
+        if (Tout) Tout[i] = T;
+    }
     return true;
 }
 

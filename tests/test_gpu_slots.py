@@ -69,10 +69,15 @@ def _rays(d, n):
 def test_march_over_slots_equals_march_through_the_accessor(name, codec):
     nvq = _nvq()
     d = _grid(nvq, _host(nvq, name), codec)
-    for n, dt in ((1, 0.5), (65, 0.37), (4097, 0.5), (4096, 1.9)):
+    for n, dt in ((1, 0.5), (65, 0.37), (4097, 0.5), (4096, 1.9), (1 << 20, 0.5), ((1 << 20) + 65, 0.37)):
         eye, dirs = _rays(d, n)
         L, T = nvq.ops.fog_march(d, eye, dirs, dt, 0.05)
         torch.cuda.synchronize()
+        if n > 1 << 18:  # around the launch size from which a ray takes one lane: larger than a capture
+            if codec == "float":  # without scratch takes, so against its first rays
+                a, b = nvq.ops.fog_march(d, eye[:4099].contiguous(), dirs[:4099].contiguous(), dt, 0.05)
+                assert torch.equal(L[:4099], a) and torch.equal(T[:4099], b)
+            continue
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             Lc, Tc = nvq.ops.fog_march(d, eye, dirs, dt, 0.05)
