@@ -320,7 +320,7 @@ struct TileOrder {
     char* withMap = nullptr; // the scratch asked for beside it, 256-byte aligned
 };
 char* acquireWithMap(WorkspaceLease& lease, const GridView& g, uint64_t rays, uint32_t parts, float iso, size_t need,
-                     SlotMap& M, bool& mapped, hipStream_t st);
+                     size_t withMap, SlotMap& M, bool& mapped, hipStream_t st);
 // With `map`, also the grid's slot map (nvq_slots.h) and `withMapBytes` of scratch, where the rule on
 // its size, the scratch and the stream allow it: a stream under graph capture takes none.
 int tileOrder(const GridView& g, const float* eye, const float* dir, const Sched& s, TileOrder& out, hipStream_t st,

@@ -278,10 +278,10 @@ __global__ __launch_bounds__(kBlock) void k_fog_march_slots(SlotMap M, GridView 
 
 // Four lanes per ray (fogMarchQuad): a wavefront takes a quarter of a tile, 4x4 pixels or 16 rays.  Up to
 // kQuadTiles tiles, where the lanes that repeat a ray's walk would otherwise be missing from the chip.
-// Rays through the 512^3 fog, one lane and four per ray: 64^2 1302 and 912 us, 512^2 1602 and 965,
-// 800^2 1370 and 1103, 1024^2 1590 and 1561, 1200^2 1908 and 1997; through the 256^3 fog 640^2 527 and 359,
-// 1024^2 704 and 674, 1200^2 803 and 870.
-constexpr uint64_t kQuadTiles = 16384;
+// One lane and four per ray through the 512^3 fog: 64^2 rays 1302 and 912 us; cameras from near to far,
+// 512^2 rays 1483 and 1229, 1757 and 1074, 1599 and 971; 640^2 1625 and 1576, 1453 and 1182, 1290 and 854;
+// 800^2 2110 and 2182, 1650 and 1621, 1373 and 1105; 1024^2 2936 and 3225, 2229 and 2382, 1594 and 1563.
+constexpr uint64_t kQuadTiles = 8192;
 template<uint32_t GT>
 __global__ __launch_bounds__(kBlock) void k_fog_march_quads(SlotMap M, GridView g, const GridView* whole,
                                                             const float* __restrict__ eye, const float* __restrict__ dir,
@@ -593,10 +593,8 @@ int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const 
     const size_t need = keyBytes + orderBytes + countBytes + extraBytes;
     char* base = nullptr;
     if (map) {
-        // what goes with the map lies before it
-        const size_t at = (need + 255) & ~size_t(255);
-        base = acquireWithMap(out.lease, g, s.n, kMapBricks, 0.0f, at + withMapBytes, *map, out.map, st);
-        out.withMap = out.map && withMapBytes ? base + at : nullptr;
+        base = acquireWithMap(out.lease, g, s.n, kMapBricks, 0.0f, need, withMapBytes, *map, out.map, st);
+        out.withMap = out.map && withMapBytes ? base + ((need + 255) & ~size_t(255)) : nullptr;
     } else if (need) {
         base = out.lease.acquire(need, st);
     }
@@ -617,20 +615,25 @@ int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const 
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// Scratch of `need` bytes plus a slot map of `parts` for `rays` rays, where the rule on the map's size, the
-// scratch and the stream allow it (mapped; the base is then need bytes, 256-aligned, before it).
+// Scratch of `need` bytes, and a slot map of `parts` for `rays` rays with `withMap` bytes beside it, where the
+// rule on the map's size, the scratch and the stream allow it (mapped).  The block holds need, withMap
+// (from the next multiple of 256 on) and the map; without a map need alone.
 char* nvq::acquireWithMap(WorkspaceLease& lease, const GridView& g, uint64_t rays, uint32_t parts, float iso, size_t need,
-                          SlotMap& M, bool& mapped, hipStream_t st)
+                          size_t withMap, SlotMap& M, bool& mapped, hipStream_t st)
 {
     mapped = false;
-    need = (need + 255) & ~size_t(255);
+    const size_t at = ((need + 255) & ~size_t(255)) + ((withMap + 255) & ~size_t(255));
     const size_t mapBytes = slotMapBytes(g, rays, parts);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     // a captured launch must not depend on scratch that a later call on the stream may replace
-    if (mapBytes && hipStreamIsCapturing(st, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone) {
-        char* base = lease.acquire(need + mapBytes, st);
+    if (mapBytes && hipStreamIsCapturing(st, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        capturing = hipStreamCaptureStatusActive;
+    }
+    if (mapBytes && capturing == hipStreamCaptureStatusNone) {
+        char* base = lease.acquire(at + mapBytes, st);
         if (base) {
-            mapped = launchSlotMap(g, base + need, M, parts, iso, st) == 0;
+            mapped = launchSlotMap(g, base + at, M, parts, iso, st) == 0;
             return base;
         }
     }
@@ -814,7 +817,7 @@ static int crossing(const nvq_grid* grid, const float* eye, const float* dir, ui
     WorkspaceLease lease;
     SlotMap M;
     bool mapped = false;
-    (void)acquireWithMap(lease, grid->view, n, kMapSigns, iso, 0, M, mapped, s);
+    (void)acquireWithMap(lease, grid->view, n, kMapSigns, iso, 0, 0, M, mapped, s);
     const Sched sc = makeSched(n, image_width);
     return launchTyped<RunZeroCrossing>(grid->view.type, grid->view, grid->dview, mapped ? &M : nullptr, eye, dir, sc, iso, o, s);
 }
@@ -830,7 +833,7 @@ int nvq_get_value(const nvq_grid* grid, const int32_t* ijk, uint64_t n, float* v
     SlotMap M;
     bool mapped = false;
     if (n >= kValueMapMin && slotCount(grid->view) <= n / 8)
-        (void)acquireWithMap(lease, grid->view, n, 0u, 0.0f, 0, M, mapped, S(stream));
+        (void)acquireWithMap(lease, grid->view, n, 0u, 0.0f, 0, 0, M, mapped, S(stream));
     return launchTyped<RunGetValue>(grid->view.type, grid->view, mapped ? &M : nullptr, ijk, n, val, active, dim, S(stream));
 }
 

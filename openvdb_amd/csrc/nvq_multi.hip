@@ -210,7 +210,11 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
     // no map on a captured stream (the launch must not depend on scratch that a later call may
     // replace), nor where the scratch cannot grow
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    any = any && hipStreamIsCapturing(s, &capturing) == hipSuccess && capturing == hipStreamCaptureStatusNone;
+    if (any && hipStreamIsCapturing(s, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        capturing = hipStreamCaptureStatusActive;
+    }
+    any = any && capturing == hipStreamCaptureStatusNone;
     WorkspaceLease lease;
     char* base = any ? lease.acquire(total, s) : nullptr;
     if (!base) {
