@@ -10,6 +10,7 @@
 #include "nvq_internal.h"
 #include "nvq_profile.h"
 #include "nvq_rays.h"
+#include "nvq_rules.h"
 
 #include <hip/hip_runtime.h>
 
@@ -118,24 +119,25 @@ __global__ __launch_bounds__(kBlock) void k_multi_again(MultiArgs A, const float
 __global__ __launch_bounds__(kBlock) void k_multi_tile_cost(MultiArgs A, const float* __restrict__ eye,
                                                             const float* __restrict__ dir, uint32_t* __restrict__ key)
 {
-    const uint32_t t = (blockIdx.x * kBlock + threadIdx.x) >> 2, corner = threadIdx.x & 3u;
+    const uint32_t corner = threadIdx.x & 3u;
+    const uint64_t tile = tileOfQuad(blockIdx.x, blockIdx.y, threadIdx.x, kBlock);
+    if (tile >= A.totalTiles) return; // whole quads
+    const uint32_t t = uint32_t(tile);
     float c = 0.0f;
-    if (t < A.totalTiles) {
-        uint32_t j = 0;
-        while (j + 1 < A.k && A.slot[j + 1].tileBase <= t) ++j;
-        const MultiSlot& S = A.slot[j];
-        const uint32_t local = t - S.tileBase;
-        const uint32_t tx = local % S.tilesX, ty = local / S.tilesX;
-        const uint32_t px = tx * 8 + (corner & 1u) * 7u, py = ty * 8 + (corner >> 1) * 7u;
-        const uint64_t i = S.rayBase + uint64_t(py) * S.width + px;
-        if (px < S.width && py < S.height && i < S.rayEnd) {
-            c = clippedLength(*S.view, eye + 3 * i, dir + 3 * i);
-            if (S.op == kOpZeroCrossing) c *= 0.0625f;
-        }
+    uint32_t j = 0;
+    while (j + 1 < A.k && A.slot[j + 1].tileBase <= t) ++j;
+    const MultiSlot& S = A.slot[j];
+    const uint32_t local = t - S.tileBase;
+    const uint32_t tx = local % S.tilesX, ty = local / S.tilesX;
+    const uint32_t px = tx * 8 + (corner & 1u) * 7u, py = ty * 8 + (corner >> 1) * 7u;
+    const uint64_t i = S.rayBase + uint64_t(py) * S.width + px;
+    if (px < S.width && py < S.height && i < S.rayEnd) {
+        c = clippedLength(*S.view, eye + 3 * i, dir + 3 * i);
+        if (S.op == kOpZeroCrossing) c *= 0.0625f;
     }
     c = fmaxf(c, __shfl_xor(c, 1));
     c = fmaxf(c, __shfl_xor(c, 2));
-    if (corner == 0 && t < A.totalTiles) key[t] = costKey(c, t);
+    if (corner == 0) key[t] = costKey(c, t);
 }
 
 constexpr int kMaxDevices = 64;
@@ -229,8 +231,8 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
     hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(kQueueBands), 0, s, counter);
     if (ordered) {
         ProfScope prof("tile_order", s);
-        hipLaunchKernelGGL(k_multi_tile_cost, dim3((A.totalTiles + kBlock / 4 - 1) / (kBlock / 4)), dim3(kBlock), 0, s, A,
-                           eye, dir, key);
+        const LaunchRows rows = quadRows(A.totalTiles, kBlock);
+        hipLaunchKernelGGL(k_multi_tile_cost, dim3(rows.x, rows.y), dim3(kBlock), 0, s, A, eye, dir, key);
         launchTileOrder(key, uint64_t(A.totalTiles), order,
                         reinterpret_cast<uint32_t*>(base + 2 * kQueueBytes + 2 * keyBytes), s);
     }
