@@ -9,7 +9,10 @@
  * queue counters, slot maps of ray queries: about 3 KB per leaf, the sort buffers of binned point
  * queries) lives in one grow-only block per (device, stream) that the library keeps until the
  * process ends; ray queries take no slot map on a stream under graph capture, or where the block
- * cannot grow, and give the same bits without it.  Besides the block, the library holds
+ * cannot grow, and give the same bits without it.  A captured call uses its stream's block as it is, or
+ * runs without scratch where that is too small, and the block it uses is kept for the graph's replays;
+ * replay such a graph on the stream it was captured on, or not beside other calls on that stream.
+ * Besides the block, the library holds
  * the opt-in kernel profiler (nvq_profile_*), the work-queue array of nvq_multi_query_noalloc and
  * a small pinned host buffer per calling thread for values it reads back.  Calls on distinct
  * streams are thread-safe; calls on one stream from several threads are serialised.  The caller

@@ -293,8 +293,10 @@ inline void launchTileOrder(const uint32_t* key, uint64_t tiles, uint32_t* order
 // once some tens of calls had run).  Calls on one stream execute in stream order, so they can
 // share the block; the lease's lock serialises host threads that issue calls on the same stream.
 // When a call needs more, the old block is freed in stream order and a larger one taken; the last
-// block of each stream is kept until the process ends.
+// block of each stream is kept until the process ends.  So is a block that a captured launch uses
+// (nvq_workspace.h); a capture on a stream whose block is too small gets none.
 struct StreamWorkspace;
+bool isCapturing(hipStream_t s); // also where the stream cannot be asked
 class WorkspaceLease {
 public:
     WorkspaceLease() = default;
@@ -304,9 +306,11 @@ public:
     // The stream's block, at least `bytes` long, held until the lease ends; nullptr on failure.
     // One lease per call: a second acquire on the same lease fails.
     char* acquire(size_t bytes, hipStream_t s);
+    bool capturing() const { return capturing_; } // the last acquire met a stream under capture
 
 private:
     StreamWorkspace* w_ = nullptr;
+    bool capturing_ = false;
 };
 
 // The longest-first order of a ray launch (nullptr up to kOrderMinTiles tiles), in the stream's
@@ -372,7 +376,8 @@ int makeMultiArgs(const nvq_grid* const* host_grids, uint32_t k, const uint64_t*
 // wavefronts in flight share one region of the grids) while the atomics are spread over 8
 // addresses instead of serialising on one.  A wavefront starts on its XCD's counter and moves to
 // the next once that counter's chunks pass the end; it returns after all 8, so every wavefront
-// exits.
+// exits.  Without counters (a captured launch that gets no scratch) the wavefronts take the tiles in
+// turn.
 constexpr uint32_t kQueueBands = 8, kQueueStride = 64, kQueueChunk = 1; // stride in uint32 (256 B)
 constexpr size_t kQueueBytes = size_t(kQueueBands) * kQueueStride * sizeof(uint32_t);
 
@@ -383,15 +388,21 @@ __device__ __forceinline__ void forEachQueuedTile(uint32_t* __restrict__ counter
     const uint32_t chunks = (total + kQueueChunk - 1) / kQueueChunk;
     for (uint32_t k = 0; k < kQueueBands; ++k) {
         const uint32_t r = (home + k) & (kQueueBands - 1);
-        for (;;) {
-            uint32_t b = 0;
-            if (lane == 0) b = atomicAdd(counters + r * kQueueStride, 1u);
-            b = __shfl(b, 0, 64);
-            const uint64_t q = uint64_t(b) * kQueueBands + r;
+        for (uint32_t i = 0;; ++i) {
+            uint64_t q;
+            if (counters) {
+                uint32_t b = 0;
+                if (lane == 0) b = atomicAdd(counters + r * kQueueStride, 1u);
+                b = __shfl(b, 0, 64);
+                q = uint64_t(b) * kQueueBands + r;
+            } else {
+                q = (uint64_t(i) * gridDim.x + blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+            }
             if (q >= chunks) break; // counter r has handed out all its chunks
             const uint32_t t0 = uint32_t(q) * kQueueChunk, t1 = t0 + kQueueChunk < total ? t0 + kQueueChunk : total;
             for (uint32_t t = t0; t < t1; ++t) f(t);
         }
+        if (!counters) break;
     }
 }
 

@@ -84,7 +84,10 @@ int launchIso(const GridView& g, const IsoCamera& c, int persistent, float* imag
               hipStream_t s)
 {
     const uint64_t n = uint64_t(c.width) * uint32_t(c.height);
-    if (!persistent) {
+    WorkspaceLease lease;
+    uint32_t* counter = persistent ? reinterpret_cast<uint32_t*>(lease.acquire(kQueueBytes, s)) : nullptr;
+    if (persistent && !counter && !lease.capturing()) return -2;
+    if (!counter) { // or recorded without scratch: the same image
         const Sched sc = makeSched(n, uint32_t(c.width));
         ProfScope prof("k_iso_render", s);
         hipLaunchKernelGGL(k_iso_render<GT>, dim3(launchBlocks(sc)), dim3(kBlock), 0, s, g, c, sc, image, hit, t);
@@ -94,9 +97,6 @@ int launchIso(const GridView& g, const IsoCamera& c, int persistent, float* imag
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         return -1;
     const uint32_t tilesX = (uint32_t(c.width) + 7) / 8, tiles = tilesX * ((uint32_t(c.height) + 7) / 8);
-    WorkspaceLease lease;
-    uint32_t* counter = reinterpret_cast<uint32_t*>(lease.acquire(kQueueBytes, s));
-    if (!counter) return -2;
     hipLaunchKernelGGL(k_queue_reset, dim3(1), dim3(kQueueBands), 0, s, counter);
     uint32_t blocks = uint32_t(cus) * 8u;
     const uint32_t wavesNeeded = (tiles + (kBlock / 64) - 1) / (kBlock / 64);

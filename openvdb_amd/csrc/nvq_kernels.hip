@@ -11,6 +11,7 @@
 #include "nvq_sample.h"
 #include "nvq_rays.h"
 #include "nvq_slots.h"
+#include "nvq_workspace.h"
 #include "../../include/nvq.h"
 
 #include <cstdlib>
@@ -537,8 +538,7 @@ hipError_t nvq::readBack(void* dst, const void* src, size_t bytes, hipStream_t s
 
 struct nvq::StreamWorkspace {
     std::mutex use;
-    char* ptr = nullptr;
-    size_t bytes = 0;
+    ScratchBlock block;
 };
 
 namespace {
@@ -563,30 +563,39 @@ char* nvq::WorkspaceLease::acquire(size_t bytes, hipStream_t s)
         w = e.get();
     }
     w->use.lock();
-    w_ = w;
-    if (w->bytes < bytes || !w->ptr) {
-        if (w->ptr) (void)hipFreeAsync(w->ptr, s); // after the earlier calls' kernels on s
-        w->ptr = nullptr;
-        w->bytes = 0;
-        const size_t want = std::max<size_t>(bytes + bytes / 8, size_t(1) << 20);
-        void* p = nullptr;
-        if (poolMalloc(&p, want, s) != hipSuccess) {
+    struct Pool {
+        hipStream_t s;
+        char* alloc(size_t want)
+        {
+            void* p = nullptr;
+            if (poolMalloc(&p, want, s) == hipSuccess) return static_cast<char*>(p);
             (void)hipGetLastError();
-            w_ = nullptr; // the caller may ask again for less
-            w->use.unlock();
             return nullptr;
         }
-        w->ptr = static_cast<char*>(p);
-        w->bytes = want;
+        void free(char* p) { (void)hipFreeAsync(p, s); } // after the earlier calls' kernels on s
+    };
+    capturing_ = isCapturing(s);
+    char* p = scratchAcquire(w->block, bytes, capturing_, Pool{s});
+    if (p) w_ = w;
+    else w->use.unlock(); // the caller may ask again for less
+    return p;
+}
+
+bool nvq::isCapturing(hipStream_t s)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
     }
-    return w->ptr;
+    return status != hipStreamCaptureStatusNone;
 }
 
 int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const Sched& s, TileOrder& out, hipStream_t st,
                    size_t extraBytes, SlotMap* map, size_t withMapBytes)
 {
     if (s.tiles == 0 || s.tiles > (uint64_t(1) << 32)) return -1;
-    const bool ordered = s.tiles > kOrderMinTiles;
+    bool ordered = s.tiles > kOrderMinTiles;
     const size_t keyBytes = ordered ? (size_t(s.tiles) * 4 + 255) & ~size_t(255) : 0;
     const size_t orderBytes = keyBytes;
     const size_t countBytes = ordered ? orderScratchBytes(s.tiles) : 0;
@@ -598,7 +607,10 @@ int nvq::tileOrder(const GridView& g, const float* eye, const float* dir, const 
     } else if (need) {
         base = out.lease.acquire(need, st);
     }
-    if (need && !base) return -1;
+    if (need && !base) {
+        if (!out.lease.capturing() || extraBytes) return -1;
+        ordered = false; // recorded without scratch: image order, the same results
+    }
     out.extra = extraBytes ? base + keyBytes + orderBytes + countBytes : nullptr;
     if (!ordered) {
         out.order = nullptr;
@@ -624,13 +636,8 @@ char* nvq::acquireWithMap(WorkspaceLease& lease, const GridView& g, uint64_t ray
     mapped = false;
     const size_t at = ((need + 255) & ~size_t(255)) + ((withMap + 255) & ~size_t(255));
     const size_t mapBytes = slotMapBytes(g, rays, parts);
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    // a captured launch must not depend on scratch that a later call on the stream may replace
-    if (mapBytes && hipStreamIsCapturing(st, &capturing) != hipSuccess) {
-        (void)hipGetLastError();
-        capturing = hipStreamCaptureStatusActive;
-    }
-    if (mapBytes && capturing == hipStreamCaptureStatusNone) {
+    // a captured launch takes the accessor, whatever scratch the stream happens to hold
+    if (mapBytes && !isCapturing(st)) {
         char* base = lease.acquire(at + mapBytes, st);
         if (base) {
             mapped = launchSlotMap(g, base + at, M, parts, iso, st) == 0;

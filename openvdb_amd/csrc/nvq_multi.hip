@@ -209,21 +209,22 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
         total += bytes[j];
         any = any || bytes[j];
     }
-    // no map on a captured stream (the launch must not depend on scratch that a later call may
-    // replace), nor where the scratch cannot grow
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (any && hipStreamIsCapturing(s, &capturing) != hipSuccess) {
-        (void)hipGetLastError();
-        capturing = hipStreamCaptureStatusActive;
-    }
-    any = any && capturing == hipStreamCaptureStatusNone;
+    // no map on a captured stream, nor where the scratch cannot grow
+    any = any && !isCapturing(s);
     WorkspaceLease lease;
     char* base = any ? lease.acquire(total, s) : nullptr;
     if (!base) {
         any = false;
         base = lease.acquire(need, s);
     }
-    if (!base) return -2;
+    const CrossingOut o{hit, ijk, a, b, normal};
+    const dim3 blocks(queryBlocks(A, cus));
+    if (!base) {
+        if (!lease.capturing()) return -2;
+        // recorded without scratch: the tiles in turn
+        hipLaunchKernelGGL(k_multi_query, blocks, dim3(kBlock), 0, s, A, eye, dir, dt, sigma, nullptr, nullptr, o);
+        return hipGetLastError() == hipSuccess ? 0 : -4;
+    }
     uint32_t* counter = reinterpret_cast<uint32_t*>(base);
     uint32_t* second = reinterpret_cast<uint32_t*>(base + kQueueBytes);
     uint32_t* key = reinterpret_cast<uint32_t*>(base + 2 * kQueueBytes);
@@ -236,8 +237,6 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
         launchTileOrder(key, uint64_t(A.totalTiles), order,
                         reinterpret_cast<uint32_t*>(base + 2 * kQueueBytes + 2 * keyBytes), s);
     }
-    const CrossingOut o{hit, ijk, a, b, normal};
-    const dim3 blocks(queryBlocks(A, cus));
     if (any) {
         uint32_t* count = reinterpret_cast<uint32_t*>(base + need);
         uint32_t* again = reinterpret_cast<uint32_t*>(base + need + 256);
