@@ -304,8 +304,8 @@ public:
     WorkspaceLease& operator=(const WorkspaceLease&) = delete;
     ~WorkspaceLease();
     // The stream's block, at least `bytes` long, held until the lease ends; nullptr on failure.
-    // One lease per call: a second acquire on the same lease fails.
-    char* acquire(size_t bytes, hipStream_t s);
+    // One block per lease: once it has one, a second acquire fails.  `optional`: the caller does without.
+    char* acquire(size_t bytes, hipStream_t s, bool optional = false);
     bool capturing() const { return capturing_; } // the last acquire met a stream under capture
 
 private:

@@ -551,7 +551,7 @@ nvq::WorkspaceLease::~WorkspaceLease()
     if (w_) w_->use.unlock();
 }
 
-char* nvq::WorkspaceLease::acquire(size_t bytes, hipStream_t s)
+char* nvq::WorkspaceLease::acquire(size_t bytes, hipStream_t s, bool optional)
 {
     int dev = 0;
     if (w_ || hipGetDevice(&dev) != hipSuccess) return nullptr;
@@ -575,7 +575,7 @@ char* nvq::WorkspaceLease::acquire(size_t bytes, hipStream_t s)
         void free(char* p) { (void)hipFreeAsync(p, s); } // after the earlier calls' kernels on s
     };
     capturing_ = isCapturing(s);
-    char* p = scratchAcquire(w->block, bytes, capturing_, Pool{s});
+    char* p = scratchAcquire(w->block, bytes, capturing_, optional, Pool{s});
     if (p) w_ = w;
     else w->use.unlock(); // the caller may ask again for less
     return p;
@@ -638,7 +638,7 @@ char* nvq::acquireWithMap(WorkspaceLease& lease, const GridView& g, uint64_t ray
     const size_t mapBytes = slotMapBytes(g, rays, parts);
     // a captured launch takes the accessor, whatever scratch the stream happens to hold
     if (mapBytes && !isCapturing(st)) {
-        char* base = lease.acquire(at + mapBytes, st);
+        char* base = lease.acquire(at + mapBytes, st, true);
         if (base) {
             mapped = launchSlotMap(g, base + at, M, parts, iso, st) == 0;
             return base;

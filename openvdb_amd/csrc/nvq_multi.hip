@@ -212,7 +212,7 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
     // no map on a captured stream, nor where the scratch cannot grow
     any = any && !isCapturing(s);
     WorkspaceLease lease;
-    char* base = any ? lease.acquire(total, s) : nullptr;
+    char* base = any ? lease.acquire(total, s, true) : nullptr;
     if (!base) {
         any = false;
         base = lease.acquire(need, s);
