@@ -37,7 +37,7 @@ namespace {
 // 128 entries 25.7, 64 entries 25.4 of an earlier form; written back every 2 steps 16.3 ms,
 // every 4 15.5, every 8 16.5; one step between looks at the wavefront's slowest ray 15.5 ms,
 // four 15.7 with a lag of 4 steps, 14.0 with 8, 14.4 with 12.
-constexpr uint32_t kCacheBlocks = 128, kCacheMisses = 64;
+constexpr uint32_t kCacheMisses = 64; // and kCacheBlocks entries
 constexpr uint32_t kCacheSteps = 4, kCacheAge = 4; // write back every kCacheSteps what is kCacheAge old
 constexpr float kCacheLag = 8.0f;                  // steps a ray may be ahead of the slowest
 constexpr uint32_t kMaxBlockLeaves = 1u << 20;
@@ -167,10 +167,6 @@ struct BlockCache {
     uint8_t list[kCacheBlocks];             // entries to write back
 };
 static_assert(kCacheBlocks <= 256, "list holds bytes");
-struct BlockBox {
-    uint32_t sx, sy;
-};
-constexpr uint32_t kNoBlock = 0xffffffffu;
 
 __device__ __forceinline__ float waveMinDpp(float x)
 {
@@ -553,21 +549,6 @@ __global__ __launch_bounds__(kBlock) void k_fixed_to_float(const long long* __re
 
 } // namespace
 
-// Strides of a block tag, at least the box's extents, with the low bits that spread best.
-static bool blockBox(const SlotMap& M, BlockBox& X)
-{
-    auto atLeast = [](uint64_t n, uint32_t low) {
-        const uint64_t r = (n & ~uint64_t(kCacheBlocks - 1)) | low;
-        return r < n ? r + kCacheBlocks : r;
-    };
-    // pos * 8 + word fits 32 bits
-    if (uint64_t(M.n[0]) * M.n[1] * M.n[2] > (1u << 23)) return false;
-    const uint64_t sy = atLeast(4ull * M.n[2], 19u), sx = atLeast(4ull * M.n[1] * sy, 45u);
-    X.sy = uint32_t(sy);
-    X.sx = uint32_t(sx);
-    return 4ull * M.n[0] * sx < kNoBlock;
-}
-
 int fogMarchBackward(const GridView& g, const float* eye, const float* dir, uint64_t n, uint32_t width, float dt,
                      float sigma, const float* L, const float* T, const float* gL, const float* gT, int64_t* accum,
                      int shift, hipStream_t s)
@@ -579,14 +560,16 @@ int fogMarchBackward(const GridView& g, const float* eye, const float* dir, uint
     // The tiled adjoint wherever the grid has a slot map and its blocks (4 KB per leaf) stay within 4 GiB:
     // it was the faster one from 1024 rays on, as an image or a scattered batch (1024 rays through a
     // 256^3 fog: accessor 7.1 ms, blocks 2.9; 1 M scattered rays 23.5 and 10.7).
+    // Decided before any of it is allocated or built.
     BlockBox X{};
-    const uint64_t blockBytes = g.leafCount && g.leafCount <= kMaxBlockLeaves && sc.tiles < (1u << 26) ? uint64_t(g.leafCount) * 4096u : 0;
-    if (tileOrder(g, eye, dir, sc, to, s, 256, blockBytes ? &M : nullptr, blockBytes) != 0) return -1;
+    const bool tiled = g.leafCount && g.leafCount <= kMaxBlockLeaves && sc.tiles < (1u << 26) && blockBoxOf(slotBoxOf(g.bbox), X);
+    const uint64_t blockBytes = tiled ? uint64_t(g.leafCount) * 4096u : 0;
+    if (tileOrder(g, eye, dir, sc, to, s, 256, tiled ? &M : nullptr, blockBytes) != 0) return -1;
     uint32_t* flag = reinterpret_cast<uint32_t*>(to.extra);
     hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, s, flag);
     unsigned long long* acc = reinterpret_cast<unsigned long long*>(accum);
     const bool index = g.type == GT_ONINDEX;
-    if (to.map && blockBox(M, X)) {
+    if (to.map) {
         unsigned long long* blocks = reinterpret_cast<unsigned long long*>(to.withMap);
         const uint64_t words = blockBytes / 16;
         hipLaunchKernelGGL(k_zero_blocks, dim3(uint32_t((words + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,

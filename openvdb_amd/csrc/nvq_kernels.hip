@@ -839,7 +839,8 @@ int nvq_get_value(const nvq_grid* grid, const int32_t* ijk, uint64_t n, float* v
     WorkspaceLease lease;
     SlotMap M;
     bool mapped = false;
-    if (n >= kValueMapMin && slotCount(grid->view) <= n / 8)
+    const uint64_t slots = n >= kValueMapMin ? slotBoxOf(grid->view.bbox).count : 0;
+    if (slots && slots <= n / 8)
         (void)acquireWithMap(lease, grid->view, n, 0u, 0.0f, 0, 0, M, mapped, S(stream));
     return launchTyped<RunGetValue>(grid->view.type, grid->view, mapped ? &M : nullptr, ijk, n, val, active, dim, S(stream));
 }

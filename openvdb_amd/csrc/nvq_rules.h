@@ -24,4 +24,51 @@ constexpr uint64_t tileOfQuad(uint32_t blockX, uint32_t blockY, uint32_t thread,
     return (uint64_t(blockY) * kRowBlocks + blockX) * (threads / 4u) + (thread >> 2);
 }
 
+// ------------------------------------------------------------------ slot tables
+// The 8^3 slots of a grid's bbox, one slot wider below and two above, so that a cell's eight corners and a
+// brick's upper neighbours stay inside.
+constexpr uint64_t kMaxMapSlots = uint64_t(1) << 24;
+struct SlotBox {
+    int32_t lo[3];  // first slot per axis
+    uint32_t n[3];  // slots per axis
+    uint64_t count; // 0: no table (an empty grid, coordinates whose neighbours could leave the int32 range, too many)
+};
+inline SlotBox slotBoxOf(const int32_t bbox[6])
+{
+    SlotBox b{};
+    uint64_t count = 1;
+    for (int a = 0; a < 3; ++a) {
+        if (bbox[a] > bbox[3 + a] || bbox[a] < -(1 << 30) || bbox[3 + a] > (1 << 30)) return b;
+        const int64_t l = (int64_t(bbox[a]) >> 3) - 1, h = (int64_t(bbox[3 + a]) >> 3) + 2;
+        b.lo[a] = int32_t(l);
+        b.n[a] = uint32_t(h - l + 1);
+        count *= b.n[a];
+        if (count > kMaxMapSlots) return b;
+    }
+    b.count = count;
+    return b;
+}
+
+// ------------------------------------------------------------------ block cache of the march's adjoint
+constexpr uint32_t kCacheBlocks = 128;
+constexpr uint32_t kNoBlock = 0xffffffffu;
+// A block's tag is its linear position in the table's box, bx * sx + by * sy + bz.
+struct BlockBox {
+    uint32_t sx, sy;
+};
+// Strides of a block tag, at least the box's extents, with the low bits that spread best.  False: no cache (a
+// position, slot * 64 + block, times 8 words would leave 32 bits, or a tag would).
+inline bool blockBoxOf(const SlotBox& b, BlockBox& x)
+{
+    auto atLeast = [](uint64_t n, uint32_t low) {
+        const uint64_t r = (n & ~uint64_t(kCacheBlocks - 1)) | low;
+        return r < n ? r + kCacheBlocks : r;
+    };
+    if (b.count == 0 || b.count > (1u << 23)) return false;
+    const uint64_t sy = atLeast(4ull * b.n[2], 19u), sx = atLeast(4ull * b.n[1] * sy, 45u);
+    x.sy = uint32_t(sy);
+    x.sx = uint32_t(sx);
+    return 4ull * b.n[0] * sx < kNoBlock;
+}
+
 } // namespace nvq

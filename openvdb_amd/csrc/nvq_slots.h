@@ -17,6 +17,7 @@
 // All values are ReadAccessor::getValue results, so the queries' outputs keep their bits.
 #pragma once
 #include "nvq_device.h"
+#include "nvq_rules.h"
 
 #include <hip/hip_runtime.h>
 
@@ -164,7 +165,7 @@ __device__ __forceinline__ bool slotTrilinear(const SlotMap& M, float px, float 
 // accessor's latency: one ray through that fog takes milliseconds, as its lookups wait for each other.
 // So small launches take a map too, up to these sizes per launch and per ray; beyond them, and
 // where a brick's offset would leave 32 bits, the accessor answers.
-constexpr uint64_t kMaxMapSlots = uint64_t(1) << 24, kMapSlotsPerRay = 256, kMapSlotsFree = 1u << 20;
+constexpr uint64_t kMapSlotsPerRay = 256, kMapSlotsFree = 1u << 20;
 constexpr uint64_t kMaxMapLeaves = 1400000, kMapLeavesPerRay = 64, kMapLeavesFree = 1u << 18;
 
 // ------------------------------------------------------------------ crossings
@@ -326,7 +327,6 @@ __device__ __forceinline__ bool isoCrossingSlots(const SlotMap& M, const GridVie
 // the table's 32-bit offsets.  launchSlotMap builds it in `mem` (256-byte aligned).
 // `parts`: kMapBricks, kMapSigns (against `iso`).
 size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts);
-uint64_t slotCount(const GridView& g); // ~0 where there is no table
 // One map of a multi-grid call: the grid's view on the host and on the device, and the memory its map
 // is built in (nullptr: none, and maps[j].entry is null).
 struct MapJob {

@@ -227,21 +227,6 @@ __global__ __launch_bounds__(kThreads) void k_maps_leaves(MapJobs J)
 
 __global__ void k_zero_word(uint32_t* p) { *p = 0u; }
 
-bool slotBox(const GridView& g, int32_t lo[3], uint32_t n[3], uint64_t& count)
-{
-    count = 1;
-    for (int a = 0; a < 3; ++a) {
-        // empty grids, and coordinates whose neighbours could leave the int32 range
-        if (g.bbox[a] > g.bbox[3 + a] || g.bbox[a] < -(1 << 30) || g.bbox[3 + a] > (1 << 30)) return false;
-        const int64_t l = (int64_t(g.bbox[a]) >> 3) - 1, h = (int64_t(g.bbox[3 + a]) >> 3) + 2;
-        lo[a] = int32_t(l);
-        n[a] = uint32_t(h - l + 1);
-        count *= n[a];
-        if (count > kMaxMapSlots) return false;
-    }
-    return true;
-}
-
 size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
 template<uint32_t GT>
@@ -257,8 +242,13 @@ void launchMap(const GridView& g, const SlotMap& M, const MapMem& W, float iso, 
 // Lays the map of g out in mem (slotMapBytes of it).
 bool layMap(const GridView& g, char* mem, uint32_t parts, SlotMap& M, MapMem& W)
 {
-    uint64_t count;
-    if (!slotBox(g, M.lo, M.n, count)) return false;
+    const SlotBox box = slotBoxOf(g.bbox);
+    const uint64_t count = box.count;
+    if (!count) return false;
+    for (int a = 0; a < 3; ++a) {
+        M.lo[a] = box.lo[a];
+        M.n[a] = box.n[a];
+    }
     const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
     auto take = [&](size_t bytes) {
         char* p = mem;
@@ -285,20 +275,10 @@ bool layMap(const GridView& g, char* mem, uint32_t parts, SlotMap& M, MapMem& W)
 
 } // namespace
 
-uint64_t slotCount(const GridView& g)
-{
-    int32_t lo[3];
-    uint32_t n[3];
-    uint64_t count;
-    return slotBox(g, lo, n, count) ? count : ~uint64_t(0);
-}
-
 size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts)
 {
-    int32_t lo[3];
-    uint32_t n[3];
-    uint64_t count;
-    if (!slotBox(g, lo, n, count)) return 0;
+    const uint64_t count = slotBoxOf(g.bbox).count;
+    if (!count) return 0;
     if (count > kMapSlotsPerRay * rays + kMapSlotsFree || g.leafCount > kMapLeavesPerRay * rays + kMapLeavesFree ||
         g.leafCount > kMaxMapLeaves)
         return 0;

@@ -40,3 +40,49 @@ def test_every_tile_has_one_quad(tmp_path, tiles):
         assert last == first + 64 * x - 1
         expect = last + 1
     assert expect - 64 * x < tiles <= expect and expect - tiles < max(64 * x if rows > 1 else 64, 64)
+
+
+BOXES = [(1, 1, 1), (4, 4, 4), (67, 67, 67), (203, 203, 203), (204, 204, 204), (255, 255, 255), (1, 1, 1 << 23),
+         (1 << 23, 1, 1), (1, 1 << 23, 1), (4096, 64, 32), (4097, 64, 32), (3, 5, 7), (32, 33, 31), (256, 256, 256)]
+
+
+@pytest.mark.parametrize("n", BOXES)
+def test_block_tags_are_distinct_and_positions_fit(tmp_path, n):
+    """blockBoxOf says before anything is built whether the adjoint's block cache can serve a box."""
+    out = run_cpp(tmp_path, f"""
+    SlotBox b{{}};
+    const uint32_t n[3] = {{{n[0]}u, {n[1]}u, {n[2]}u}};
+    b.count = 1;
+    for (int a = 0; a < 3; ++a) {{ b.n[a] = n[a]; b.count *= n[a]; }}
+    BlockBox x{{}};
+    const bool ok = blockBoxOf(b, x);
+    std::printf("%d %u %u\\n", ok ? 1 : 0, x.sx, x.sy);""")
+    ok, sx, sy = map(int, out[0].split())
+    slots = n[0] * n[1] * n[2]
+    assert not ok or slots <= 1 << 23
+    if ok:
+        assert sy >= 4 * n[2] and sx >= 4 * n[1] * sy     # distinct tags
+        assert (4 * n[0] - 1) * sx + (4 * n[1] - 1) * sy + 4 * n[2] - 1 < (1 << 32) - 2
+        assert ((slots - 1) * 64 + 63) * 8 + 7 < 1 << 32  # positions
+        assert sy % 128 == 19 and sx % 128 == 45
+    else:
+        assert slots > 1 << 22 or max(n) > 4096  # only large or very long boxes are turned away
+
+
+@pytest.mark.parametrize("bbox,n", [((0, 0, 0, 0, 0, 0), (4, 4, 4)), ((-1, 0, 7, 8, 7, 8), (6, 4, 5)),
+                                    ((5, 0, 0, 4, 9, 9), None), ((-(1 << 30), 0, 0, -(1 << 30) + 7, 7, 7), (4, 4, 4)),
+                                    ((-(1 << 30) - 1, 0, 0, 0, 7, 7), None), ((0, 0, 0, (1 << 30) + 1, 7, 7), None),
+                                    ((0, 0, 0, 2015, 2015, 2015), (255, 255, 255)),
+                                    ((0, 0, 0, 2023, 2023, 2023), (256, 256, 256)),
+                                    ((0, 0, 0, 2031, 2023, 2023), None)])
+def test_slot_box(tmp_path, bbox, n):
+    out = run_cpp(tmp_path, f"""
+    const int32_t bbox[6] = {{{", ".join(map(str, bbox))}}};
+    const SlotBox b = slotBoxOf(bbox);
+    std::printf("%llu %u %u %u %d %d %d\\n", (unsigned long long)b.count, b.n[0], b.n[1], b.n[2], b.lo[0], b.lo[1], b.lo[2]);""")
+    count, *rest = map(int, out[0].split())
+    if n is None:
+        assert count == 0
+    else:
+        assert tuple(rest[:3]) == n and count == n[0] * n[1] * n[2]
+        assert [8 * x for x in rest[3:]] == [(x & ~7) - 8 for x in bbox[:3]]
