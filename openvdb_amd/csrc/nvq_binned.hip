@@ -530,10 +530,11 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample(GridView g, BinLayou
         const float p[3] = {t.x, t.y, t.z};
         const float fx = floorf(p[0]), fy = floorf(p[1]), fz = floorf(p[2]);
         const int32_t ci = int32_t(fx) - o[0], cj = int32_t(fy) - o[1], ck = int32_t(fz) - o[2];
-        // the block [cell-1, cell+2]^3 lies in the brick iff the cell is in [1, kBrick-4]; FD6 samples that
-        // round out of the block go to the list too
+        // the block [cell-1, cell+2]^3 lies in the brick iff the cell is in [1, kBrick-4], and so do the cells of FD6
+        // samples that round out of the block (fd6Near)
+        const bool near = adjointInBlock(p, mode);
         if (valid && (uint32_t(ci - 1) > uint32_t(kBrick - 5) || uint32_t(cj - 1) > uint32_t(kBrick - 5) ||
-                      uint32_t(ck - 1) > uint32_t(kBrick - 5) || !adjointInBlock(p, mode))) {
+                      uint32_t(ck - 1) > uint32_t(kBrick - 5) || !(near || fd6Near(p)))) {
             spill[atomicAdd(spillCount, 1u)] = id;
             valid = false;
         }
@@ -542,6 +543,10 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample(GridView g, BinLayou
             const float* c0 = brick + (ci * kBrick + cj) * kBrick + ck;
             out = sampleFromBlock([&](int x, int y, int z) { return c0[(x * kBrick + y) * kBrick + z]; }, p, wantNN, wantVal,
                                   mode, k);
+            if (!near) // the gradient again, from the cells its samples lie in
+                sampleFd6Cells([&](int32_t x, int32_t y, int32_t z) {
+                    return brick[((x - o[0]) * kBrick + (y - o[1])) * kBrick + (z - o[2])];
+                }, p, k, out.g);
         }
         storeRecQuad(rec, valid, id, out.nn, out.val, out.g);
     }

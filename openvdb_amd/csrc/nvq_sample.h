@@ -159,6 +159,43 @@ __host__ __device__ __forceinline__ bool adjointInBlock(const float p[3], int mo
     return ok;
 }
 
+// FD6 samples outside the block still start in [cell-1, cell+2], so that their corners lie in [cell-1, cell+3],
+// below 2^23: p + 1 or p - 1 rounds up to the next whole number where p lies just under a power of two (or
+// just under 0), never down past one.  Ordinary inputs hold such points in numbers: lattices whose
+// spacing or map rounds a whole coordinate down.  False: NaN and larger coordinates, whose samples can
+// land on either side.
+__host__ __device__ __forceinline__ bool fd6Near(const float p[3])
+{
+    return fabsf(p[0]) < 8388608.0f && fabsf(p[1]) < 8388608.0f && fabsf(p[2]) < 8388608.0f;
+}
+
+// The FD6 gradient with each sample from its own cell, sampleEval's operations in their order; at(x, y, z) is
+// the voxel's value.  One axis at a time: for the lanes whose samples leave the block.
+template<class At>
+__device__ __forceinline__ void sampleFd6Cells(At&& at, const float p[3], const SampleConsts& k, float grad[3])
+{
+    grad[0] = grad[1] = grad[2] = 0.0f;
+#pragma unroll 1
+    for (int axis = 0; axis < 3; ++axis) {
+        float f[2];
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const float d = side ? -1.0f : 1.0f;
+            const float q0 = p[0] + (axis == 0 ? d : 0.0f), q1 = p[1] + (axis == 1 ? d : 0.0f), q2 = p[2] + (axis == 2 ? d : 0.0f);
+            const float x = floorf(q0), y = floorf(q1), z = floorf(q2);
+            Cell C;
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                C.v[s >> 2][(s >> 1) & 1][s & 1] = at(int32_t(x) + (s >> 2), int32_t(y) + ((s >> 1) & 1), int32_t(z) + (s & 1));
+            f[side] = trilerp(C, q0 - x, q1 - y, q2 - z);
+        }
+        const float g = (f[0] - f[1]) * (axis == 0 ? k.fdx : (axis == 1 ? k.fdy : k.fdz));
+        grad[0] = axis == 0 ? g : grad[0];
+        grad[1] = axis == 1 ? g : grad[1];
+        grad[2] = axis == 2 ? g : grad[2];
+    }
+}
+
 // ------------------------------------------------------------------ staged queries
 // The 8^3 slots that the block [cell-1, cell+2]^3 of a query overlaps (one or two per axis), resolved
 // to their leaf or tile value in four stages (root, upper, lower, voxels), every load of a stage in

@@ -67,3 +67,38 @@ def test_staged_adjoint(oracle, grids, n):
             want, over = oracle.sample_bwd_fixed(hosts[name], p, gn, gv, gg, mode, shift=40)
             assert not over
             assert np.array_equal(acc.cpu().numpy(), np.asarray(want).reshape(-1)), (name, mode)
+
+
+def _off_block(d, n):
+    """Points whose FD6 samples round out of their block: a coordinate just under a power of two or just under 0."""
+    r = np.random.default_rng(n + 1)
+    lo, hi = np.array(d.index_bbox[:3], np.float64), np.array(d.index_bbox[3:], np.float64) + 1
+    p = (r.random((n, 3)) * (hi - lo + 8) + lo - 4).astype(np.float32)
+    under = np.nextafter(np.float32([1, 2, 4, 8, 16, 32, 64]), np.float32(0))
+    under = np.concatenate([under, np.float32([-1e-9, -3e-8, -1e-30]), np.nextafter(-under, np.float32(-1e9))])
+    for a in range(3):
+        k = slice(a * n // 4, (a + 1) * n // 4)  # whole wavefronts of them, on each axis
+        p[k, a] = r.choice(under, len(p[k]))
+    k = slice(3 * n // 4, 7 * n // 8)  # some lanes of a wavefront, any axes
+    p[k] = np.where(r.random((len(p[k]), 3)) < 0.15, r.choice(under, (len(p[k]), 3)), p[k])
+    return p
+
+
+@pytest.mark.parametrize("name", ["torus", "fog_near", "torus_fp8", "torus_fpn", "far"])
+@pytest.mark.parametrize("n", [5003, (1 << 20) + 37])
+def test_queries_off_their_block(oracle, grids, name, n):
+    """Staged (small) and binned (large) batches of them; `far` lies beyond 2^24, where p +- 1 can also land two
+    cells away."""
+    nvq, hosts = grids
+    host = hosts.get(name)
+    if name == "far":
+        host = nvq.tools.create_level_set_sphere(60.0, (16777216.0 + 128.0, 0.0, 0.0), 1.0, 3.0)
+    elif name == "fog_near":
+        host = nvq.tools.create_fog_fbm([-40, -30, -20, 70, 64, 90], seed=5, amplitude=8.0)
+    d = nvq.DeviceGrid(host)
+    p = _off_block(d, n)
+    if name == "far":
+        p[:, 0] = 16777216.0 + 2.0 * np.random.default_rng(2).integers(30, 96, n)
+    got = nvq.ops.sample(d, torch.from_numpy(p).cuda(), grad_mode=1)
+    for a, b in zip(got, oracle.sample(host, p, grad_mode=1)):
+        assert np.array_equal(a.cpu().numpy().view(np.uint32), np.ascontiguousarray(b).view(np.uint32))

@@ -3,6 +3,7 @@ ends of the ranges that the entry points admit."""
 import os
 import subprocess
 
+import numpy as np
 import pytest
 
 from conftest import ROOT
@@ -86,3 +87,22 @@ def test_slot_box(tmp_path, bbox, n):
     else:
         assert tuple(rest[:3]) == n and count == n[0] * n[1] * n[2]
         assert [8 * x for x in rest[3:]] == [(x & ~7) - 8 for x in bbox[:3]]
+
+
+def test_fd6_samples_below_2_23_stay_near_their_block():
+    """fd6Near: for |p| < 2^23, floor(p + 1) and floor(p - 1) in FP32 are the next cells or one further up, so
+    that the samples' corners lie in [cell-1, cell+3]; and those slots are the ones the block itself overlaps."""
+    whole = np.unique(np.concatenate([np.arange(0, 4200), 2 ** np.arange(0, 24), 2 ** np.arange(1, 24) - 1,
+                                      2 ** np.arange(0, 23) + 1, np.random.default_rng(0).integers(0, 1 << 23, 20000)]))
+    at = np.concatenate([whole, -whole]).astype(np.float32)
+    bits = at.view(np.int32)[:, None] + np.arange(-40, 41, dtype=np.int32)
+    p = np.concatenate([bits.view(np.float32).reshape(-1), np.float32(2.0) ** -np.arange(1, 140, dtype=np.float32),
+                        -(np.float32(2.0) ** -np.arange(1, 140, dtype=np.float32))]).astype(np.float32)
+    p = p[np.isfinite(p) & (np.abs(p) < 8388608.0)]
+    cell = np.floor(p).astype(np.int64)
+    up, down = (np.floor(p + np.float32(d)).astype(np.int64) - cell for d in (1, -1))
+    assert set(np.unique(up)) == {1, 2} and set(np.unique(down)) == {-1, 0}
+    off = (up == 2) | (down == 0)
+    assert off.sum() > 100
+    first, last, far = (cell - 1) >> 3, (cell + 2) >> 3, (cell + up + 1) >> 3
+    assert np.all((far == first) | (far == last))
