@@ -563,12 +563,13 @@ __global__ __launch_bounds__(kThreads) void k_sample_list(GridView g, const floa
         const uint32_t j = base + (threadIdx.x & 63u);
         const bool valid = j < m;
         uint32_t id = 0;
-        float p[3] = {0.0f, 0.0f, 0.0f};
+        float p[3];
+        SampleOut r{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
         if (valid) {
             id = list[j];
             loadPoint(g, xyz, id, world, p);
+            r = samplePoint<GT>(g, p, wantNN, wantVal, mode, k);
         }
-        const SampleOut r = sampleWave<GT>(g, valid, p, wantNN, wantVal, mode, k);
         storeRecQuad(rec, valid, id, r.nn, r.val, r.g);
     }
 }

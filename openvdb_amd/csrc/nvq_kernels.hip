@@ -140,28 +140,19 @@ __global__ __launch_bounds__(kBlock) void k_get_value_slots(SlotMap M, GridView 
 }
 
 // ------------------------------------------------------------------ point sampling
-// 171 VGPRs uncapped (2 wavefronts per SIMD); at 4 (128, a 124-byte spill) 300,007 queries take 58.8 us
-// instead of 64.2, 1000 take 12.4 instead of 12.1.  Bound by the L1's line rate for the larger, by the
-// chain of five lookups for the smaller.
+// 4 wavefronts per SIMD (128 VGPRs, a spill of 56 to 116 bytes): 300,007 queries take 54.6 us, 1000 take 11.7.
+// Uncapped (171 VGPRs, 2 wavefronts) an earlier form took 64.2 instead of 58.8, and 12.1 instead of 12.4.
+// Bound by the L1's line rate for the larger, by the chain of five lookups for the smaller.
 template<uint32_t GT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_sample(GridView g, const float* __restrict__ xyz, uint64_t n, int world,
                                                    float* __restrict__ nn, float* __restrict__ val,
                                                    float* __restrict__ grad, int mode, SampleConsts k)
 {
     const uint64_t stride = uint64_t(gridDim.x) * kBlock;
-    // whole wavefronts, up to the last
-    for (uint64_t base = uint64_t(blockIdx.x) * kBlock + (threadIdx.x & ~63u); base < n; base += stride) {
-        const uint64_t i = base + (threadIdx.x & 63u);
-        const bool valid = i < n;
-        float p[3] = {0.0f, 0.0f, 0.0f};
-        if (valid) {
-            p[0] = xyz[3 * i];
-            p[1] = xyz[3 * i + 1];
-            p[2] = xyz[3 * i + 2];
-            if (world) worldToIndexF64(g, p);
-        }
-        const SampleOut r = sampleWave<GT>(g, valid, p, nn != nullptr, val != nullptr, grad ? mode : 0, k);
-        if (!valid) continue;
+    for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < n; i += stride) {
+        float p[3] = {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2]};
+        if (world) worldToIndexF64(g, p);
+        const SampleOut r = samplePoint<GT>(g, p, nn != nullptr, val != nullptr, grad ? mode : 0, k);
         if (nn) nn[i] = r.nn;
         if (val) val[i] = r.val;
         if (grad) {

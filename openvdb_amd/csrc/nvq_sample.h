@@ -422,81 +422,34 @@ __device__ __forceinline__ SampleOut sampleFromBlock(At&& at, const float p[3], 
     return r;
 }
 
-// Over resolved slots, for queries adjointInBlock.  False: through the accessor.
+// Over resolved slots.  FD6 samples off the block (fd6Near) read the same slots, one axis at a time.
+// False: through the accessor.
 template<uint32_t GT>
 __device__ __forceinline__ bool sampleStaged(const GridView& g, const float p[3], bool wantNN, bool wantVal, int mode,
                                              const SampleConsts& k, SampleOut& r)
 {
     const int32_t i0 = int32_t(floorf(p[0])), j0 = int32_t(floorf(p[1])), k0 = int32_t(floorf(p[2]));
     const int32_t ri = int32_t(rintf(p[0])) - i0, rj = int32_t(rintf(p[1])) - j0, rk = int32_t(rintf(p[2])) - k0;
+    const bool near = adjointInBlock(p, mode);
     BlockSlots B;
-    if (((ri | rj | rk) & ~1) || !resolveBlock<GT>(g, i0, j0, k0, false, B)) return false;
+    if (((ri | rj | rk) & ~1) || !(near || fd6Near(p)) || !resolveBlock<GT>(g, i0, j0, k0, false, B)) return false;
     r = sampleFromBlock([&](int x, int y, int z) { return blockVoxel<GT>(g, B, i0 + x, j0 + y, k0 + z); }, p, wantNN,
                         wantVal, mode, k);
+    if (!near)
+        sampleFd6Cells([&](int32_t x, int32_t y, int32_t z) { return blockVoxel<GT>(g, B, x, y, z); }, p, k, r.g);
     return true;
 }
 
-// FD6 queries whose p +- 1 rounds into a farther cell, about one in a million: the wavefront evaluates
-// them one after the other, lane 8 t + c fetching corner c of sample t (0: the value, 1..6: +x, -x, +y,
-// -y, +z, -z) and lane 56 the nearest voxel.  One such lane going through sampleEval held its whole
-// wavefront for 60 us.  Every lane of the wavefront calls this; `mine` marks the queries.
+// One query per lane.
 template<uint32_t GT>
-__device__ __forceinline__ void sampleOffBlock(const GridView& g, bool mine, const float p[3], bool wantNN, bool wantVal,
-                                               const SampleConsts& k, SampleOut& r)
-{
-    const uint32_t lane = threadIdx.x & 63u;
-    uint64_t todo = __ballot(mine);
-    while (todo) {
-        const int src = __builtin_ctzll(todo);
-        todo &= todo - 1u;
-        const float P[3] = {__shfl(p[0], src, 64), __shfl(p[1], src, 64), __shfl(p[2], src, 64)};
-        const uint32_t t = lane >> 3, c = lane & 7u;
-        // the forward's own sums: p + (+-1 along one axis, +-0 along the others)
-        float q[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float d = t != 0 && uint32_t(a) == (t - 1u) >> 1 ? 1.0f : 0.0f;
-            q[a] = t == 0 ? P[a] : ((t & 1u) ? P[a] + d : P[a] - d);
-        }
-        const float fx = floorf(q[0]), fy = floorf(q[1]), fz = floorf(q[2]);
-        int32_t x = int32_t(fx) + int32_t(c >> 2), y = int32_t(fy) + int32_t((c >> 1) & 1u), z = int32_t(fz) + int32_t(c & 1u);
-        if (t == 7u) {
-            x = int32_t(rintf(P[0]));
-            y = int32_t(rintf(P[1]));
-            z = int32_t(rintf(P[2]));
-        }
-        Accessor<GT> acc(g);
-        const float v = acc.probe(x, y, z).value;
-        Cell C;
-        const int first = int(lane & ~7u);
-#pragma unroll
-        for (int s = 0; s < 8; ++s) C.v[s >> 2][(s >> 1) & 1][s & 1] = __shfl(v, first + s, 64);
-        const float f = trilerp(C, q[0] - fx, q[1] - fy, q[2] - fz);
-        const float val = __shfl(f, 0, 64), nn = __shfl(v, 56, 64);
-        const float d[3] = {__shfl(f, 8, 64) - __shfl(f, 16, 64), __shfl(f, 24, 64) - __shfl(f, 32, 64),
-                            __shfl(f, 40, 64) - __shfl(f, 48, 64)};
-        if (int(lane) == src) {
-            r.nn = wantNN ? nn : 0.0f;
-            r.val = wantVal ? val : 0.0f;
-            r.g[0] = d[0] * k.fdx;
-            r.g[1] = d[1] * k.fdy;
-            r.g[2] = d[2] * k.fdz;
-        }
-    }
-}
-
-// One query per lane; every lane of the wavefront calls this, `valid` or not.
-template<uint32_t GT>
-__device__ __forceinline__ SampleOut sampleWave(const GridView& g, bool valid, const float p[3], bool wantNN, bool wantVal,
-                                                int mode, const SampleConsts& k)
+__device__ __forceinline__ SampleOut samplePoint(const GridView& g, const float p[3], bool wantNN, bool wantVal, int mode,
+                                                 const SampleConsts& k)
 {
     SampleOut r{0.0f, 0.0f, {0.0f, 0.0f, 0.0f}};
-    const bool off = valid && !adjointInBlock(p, mode);
-    if (valid && !off && !sampleStaged<GT>(g, p, wantNN, wantVal, mode, k, r)) {
+    if (!sampleStaged<GT>(g, p, wantNN, wantVal, mode, k, r)) {
         Accessor<GT> acc(g);
         r = sampleEval(acc, p, wantNN, wantVal, mode, k);
     }
-    if (__any(off)) sampleOffBlock<GT>(g, off, p, wantNN, wantVal, k, r);
     return r;
 }
 
