@@ -143,7 +143,9 @@ __host__ __device__ __forceinline__ void fd6Points(const float p[3], float q[6][
 
 // True when every voxel the query's terms reach lies in the plus-shaped block around its cell
 // (cell + [-1, 2] on one axis, cell + [0, 1] on the others): always, except for FD6 sample points
-// whose p +- 1 rounds into a cell other than the neighbouring one.
+// whose p +- 1 rounds into a cell other than the neighbouring one.  The cells' difference is taken, which is
+// exact where it is one: floorf(p) + 1 rounds as p + 1 does, so that from 2^24 on the two agree on
+// any cell.
 __host__ __device__ __forceinline__ bool adjointInBlock(const float p[3], int mode)
 {
     if (mode != 1) return true;
@@ -153,8 +155,7 @@ __host__ __device__ __forceinline__ bool adjointInBlock(const float p[3], int mo
 #pragma unroll
     for (int t = 0; t < 6; ++t) {
         const int ax = t >> 1;
-        const float expect = floorf(p[ax]) + ((t & 1) ? -1.0f : 1.0f);
-        ok = ok && floorf(q[t][ax]) == expect;
+        ok = ok && floorf(q[t][ax]) - floorf(p[ax]) == ((t & 1) ? -1.0f : 1.0f);
     }
     return ok;
 }

@@ -102,3 +102,33 @@ def test_queries_off_their_block(oracle, grids, name, n):
     got = nvq.ops.sample(d, torch.from_numpy(p).cuda(), grad_mode=1)
     for a, b in zip(got, oracle.sample(host, p, grad_mode=1)):
         assert np.array_equal(a.cpu().numpy().view(np.uint32), np.ascontiguousarray(b).view(np.uint32))
+
+
+def _far(nvq, x):
+    """A grid around x = `x` whose voxels all differ: at 2^24 and beyond, p + 1 and p - 1 round to even voxels."""
+    g = nvq.tools.create_level_set_sphere(60.0, (x + 128.0, 0.0, 0.0), 1.0, 3.0)
+    off, count = 672 + int(np.frombuffer(g, np.int64, 1, 672)[0]), int(np.frombuffer(g, np.uint32, 1, 704)[0])
+    leaves = g[off:off + 2144 * count].reshape(-1, 2144)
+    leaves[:, 96:] = np.random.default_rng(8).normal(size=(count, 512)).astype(np.float32).view(np.uint8)
+    return g
+
+
+@pytest.mark.parametrize("x", [2.0 ** 23, 2.0 ** 24, 2.0 ** 25])
+@pytest.mark.parametrize("n", [5003, (1 << 20) + 37])
+def test_queries_beyond_the_exact_range(oracle, grids, x, n):
+    nvq = grids[0]
+    host = _far(nvq, x)
+    d = nvq.DeviceGrid(host)
+    r = np.random.default_rng(3)
+    p = r.uniform([60, -64, -64], [196, 64, 64], (n, 3))
+    p = (p + [x, 0.0, 0.0]).astype(np.float32)
+    for mode in (1, 2, 3):
+        got = nvq.ops.sample(d, torch.from_numpy(p).cuda(), grad_mode=mode)
+        for a, b in zip(got, oracle.sample(host, p, grad_mode=mode)):
+            assert np.array_equal(a.cpu().numpy().view(np.uint32), np.ascontiguousarray(b).view(np.uint32)), mode
+    gn, gv, gg = (r.normal(size=s).astype(np.float32) for s in ((n,), (n,), (n, 3)))
+    for mode in (1, 2, 3):
+        acc = nvq.ops.sample_backward(d, torch.from_numpy(p).cuda(), *(torch.from_numpy(a).cuda() for a in (gn, gv, gg)), mode)
+        want, over = oracle.sample_bwd_fixed(host, p, gn, gv, gg, mode, shift=40)
+        assert not over
+        assert np.array_equal(acc.cpu().numpy(), np.asarray(want).reshape(-1)), mode
