@@ -1,10 +1,21 @@
 """Ray queries recorded into a graph: on a stream without scratch, and on one whose scratch block a later call
 replaces by a larger one.  Every replay against the eager call, bit for bit, with eager work between the replays."""
+import gc
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(autouse=True)
+def _no_collection_while_recording():
+    """A DeviceGrid that the collector frees waits for the device, which ends a capture: collect before, not then."""
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()
 
 RAYS = (1 << 19) + 65  # 8194 tiles: the march takes them longest first, which needs scratch
 

@@ -7,11 +7,22 @@ Covered: every codec, active tiles, leaves and nodes under render-skip flags (wh
 the accessor), bboxes that start and end inside a leaf, steps that round off their slot, rays that
 start inside, run along an axis or miss, and launches of one ray up to several tiles.
 """
+import gc
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(autouse=True)
+def _no_collection_while_recording():
+    """A DeviceGrid that the collector frees waits for the device, which ends a capture: collect before, not then."""
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()
 
 
 def _nvq():
