@@ -794,9 +794,10 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample_bwd(GridView g, BinL
         const float p[3] = {t.x, t.y, t.z};
         const int32_t ci = int32_t(floorf(p[0])) - o[0], cj = int32_t(floorf(p[1])) - o[1],
                       ck = int32_t(floorf(p[2])) - o[2];
-        // the block [cell-1, cell+2] must lie in the brick and the FD6 cells where the block expects them
+        // the block [cell-1, cell+2] must lie in the brick and the FD6 cells in it or next to it
+        const bool near = adjointInBlock(p, mode);
         if (uint32_t(ci - 1) > uint32_t(kBrick - 5) || uint32_t(cj - 1) > uint32_t(kBrick - 5) ||
-            uint32_t(ck - 1) > uint32_t(kBrick - 5) || !adjointInBlock(p, mode)) {
+            uint32_t(ck - 1) > uint32_t(kBrick - 5) || !(near || fd6Near(p))) {
             spill[atomicAdd(spillCount, 1u)] = id;
             continue;
         }
@@ -805,7 +806,8 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_sample_bwd(GridView g, BinL
             if (v != 0)
                 atomicAdd(&brick[((x - o[0]) * kBrick + (y - o[1])) * kBrick + (z - o[2])], static_cast<unsigned long long>(v));
         };
-        sampleAdjointBlock(p, d, mode, k, emit);
+        if (near) sampleAdjointBlock(p, d, mode, k, emit);
+        else sampleAdjointNear(p, d, k, emit);
     }
     if (!ok) bad = 1;
     __syncthreads();

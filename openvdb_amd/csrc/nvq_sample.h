@@ -487,8 +487,7 @@ __device__ __forceinline__ long long toFixedSat(float x, bool& ok)
     return x > 0.0f ? (1ll << 62) : -(1ll << 62);
 }
 
-// General form of the sums, for FD6 sample cells that are not the ones next to the query's cell (float
-// rounding of p +- 1): the whole wavefront takes one query, lane 8 t + c holding corner c of term t.
+// General form of the sums, for FD6 sample cells anywhere (coordinates from 2^23 on): the whole wavefront takes one query, lane 8 t + c holding corner c of term t.
 // Terms are numbered in the contract's order, so a voxel's sum is that of its lanes in lane order, and
 // its first lane emits it.  (One lane looping over all pairs of corners took 330 us.)
 // emit(x, y, z, contribution).  Every lane calls this with the same query.
@@ -546,6 +545,55 @@ __device__ __forceinline__ void sampleAdjointWave(const float p[3], const Sample
         }
     }
     if (first) emit(x, y, z, sum);
+}
+
+// The same sums where the FD6 cells are off the block but near it (fd6Near): the voxels they reach are the
+// cell's eight and, per axis, the layers at -1, 2 and 3, which only that axis's two samples reach.  One
+// voxel at a time, its terms in order.
+template<class Emit>
+__device__ __forceinline__ void sampleAdjointNear(const float p[3], const SampleGrad& d, const SampleConsts& k, Emit& emit)
+{
+    int32_t cell[3], nearest[3], o[6]; // o: cell of a sample along its axis, from `cell`
+    float f[3], q[6][3], s[6], a[6];
+    const float fd[3] = {k.fdx, k.fdy, k.fdz};
+    fd6Points(p, q);
+#pragma unroll
+    for (int b = 0; b < 3; ++b) {
+        const float whole = floorf(p[b]);
+        cell[b] = int32_t(whole);
+        f[b] = p[b] - whole;
+        nearest[b] = int32_t(rintf(p[b])) - cell[b];
+    }
+#pragma unroll
+    for (int t = 0; t < 6; ++t) {
+        const float whole = floorf(q[t][t >> 1]), s0 = d.gg[t >> 1] * fd[t >> 1];
+        o[t] = int32_t(whole) - cell[t >> 1];
+        a[t] = q[t][t >> 1] - whole;
+        s[t] = (t & 1) ? -s0 : s0;
+    }
+    auto weight = [](float frac, int32_t side) { return side ? frac : 1.0f - frac; };
+#pragma unroll 1
+    for (uint32_t v = 0; v < 44u; ++v) {
+        // voxels 0..7: the cell's; 8 + 12 axis + 4 layer + side: on the layers
+        const uint32_t w = v - 8u, axis = v < 8u ? 3u : w / 12u, layer = (w >> 2) % 3u;
+        const int32_t far = layer == 0 ? -1 : int32_t(layer) + 1, hi = int32_t(v >> 1) & 1, lo = int32_t(v) & 1;
+        const int32_t e[3] = {axis == 0 ? far : (axis == 3 ? int32_t(v >> 2) : hi), axis == 1 ? far : (axis == 2 ? lo : hi),
+                              axis == 2 ? far : lo};
+        const int32_t x[3] = {axis == 0 ? 0 : e[0], axis == 1 ? 0 : e[1], axis == 2 ? 0 : e[2]}; // sides of the other axes
+        float sum = 0.0f;
+        if (axis == 3u && d.gv != 0.0f) sum += ((d.gv * weight(f[0], x[0])) * weight(f[1], x[1])) * weight(f[2], x[2]);
+#pragma unroll
+        for (int t = 0; t < 6; ++t) {
+            const uint32_t ax = uint32_t(t) >> 1;
+            const int32_t side = e[ax] - o[t];
+            if (s[t] == 0.0f || (axis != 3u && axis != ax) || uint32_t(side) > 1u) continue;
+            const float wx = ax == 0 ? weight(a[t], side) : weight(f[0], x[0]), wy = ax == 1 ? weight(a[t], side) : weight(f[1], x[1]),
+                        wz = ax == 2 ? weight(a[t], side) : weight(f[2], x[2]);
+            sum += ((s[t] * wx) * wy) * wz;
+        }
+        if (d.gn != 0.0f && e[0] == nearest[0] && e[1] == nearest[1] && e[2] == nearest[2]) sum += d.gn;
+        emit(cell[0] + e[0], cell[1] + e[1], cell[2] + e[2], sum);
+    }
 }
 
 // Block form of the same sums (requires adjointInBlock): 32 register accumulators at constant
@@ -652,7 +700,7 @@ __device__ __forceinline__ void sampleAdjointLanes(const GridView& g, bool valid
         const int64_t key = adjointKey<GT>(g, acc.probe(x, y, z));
         if (key >= 0) atomicAdd(accum + key, static_cast<unsigned long long>(q));
     };
-    const bool off = valid && !adjointInBlock(p, mode);
+    const bool near = adjointInBlock(p, mode), off = valid && !near && !fd6Near(p);
     if (valid && !off) {
         BlockSlots B;
         if (resolveBlock<GT>(g, int32_t(floorf(p[0])), int32_t(floorf(p[1])), int32_t(floorf(p[2])), true, B)) {
@@ -668,9 +716,12 @@ __device__ __forceinline__ void sampleAdjointLanes(const GridView& g, bool valid
                     key = leaf != kNoLeaf ? int64_t(leaf / 67u) * 512 + n : -1;
                 if (key >= 0) atomicAdd(accum + key, static_cast<unsigned long long>(q));
             };
-            sampleAdjointBlock(p, d, mode, k, staged);
-        } else {
+            if (near) sampleAdjointBlock(p, d, mode, k, staged);
+            else sampleAdjointNear(p, d, k, staged);
+        } else if (near) { // a cell whose block's slots are not resolved: beyond the range of fd6Near, or odd leaves
             sampleAdjointBlock(p, d, mode, k, emit);
+        } else {
+            sampleAdjointNear(p, d, k, emit);
         }
     }
     uint64_t todo = __ballot(off);

@@ -132,3 +132,28 @@ def test_queries_beyond_the_exact_range(oracle, grids, x, n):
         want, over = oracle.sample_bwd_fixed(host, p, gn, gv, gg, mode, shift=40)
         assert not over
         assert np.array_equal(acc.cpu().numpy(), np.asarray(want).reshape(-1)), mode
+
+
+@pytest.mark.parametrize("name", ["torus", "fog_near", "far"])
+@pytest.mark.parametrize("n", [5003, (1 << 20) + 37])
+def test_adjoint_off_their_block(oracle, grids, name, n):
+    nvq, hosts = grids
+    if name == "far":
+        host = nvq.tools.create_level_set_sphere(60.0, (16777216.0 + 128.0, 0.0, 0.0), 1.0, 3.0)
+    elif name == "fog_near":
+        host = nvq.tools.create_fog_fbm([-40, -30, -20, 70, 64, 90], seed=5, amplitude=8.0)
+    else:
+        host = hosts[name]
+    d = nvq.DeviceGrid(host)
+    p = _off_block(d, n)
+    if name == "far":
+        p[:, 0] = 16777216.0 + 2.0 * np.random.default_rng(2).integers(30, 96, n)
+    r = np.random.default_rng(n)
+    gn, gv, gg = (r.normal(size=s).astype(np.float32) for s in ((n,), (n,), (n, 3)))
+    gv[::3] = 0.0
+    gn[::4] = 0.0
+    gg[::5] = 0.0
+    acc = nvq.ops.sample_backward(d, torch.from_numpy(p).cuda(), *(torch.from_numpy(a).cuda() for a in (gn, gv, gg)), 1)
+    want, over = oracle.sample_bwd_fixed(host, p, gn, gv, gg, 1, shift=40)
+    assert not over
+    assert np.array_equal(acc.cpu().numpy(), np.asarray(want).reshape(-1))
