@@ -40,6 +40,15 @@ namespace {
 constexpr uint32_t kCacheMisses = 64; // and kCacheBlocks entries
 constexpr uint32_t kCacheSteps = 4, kCacheAge = 4; // write back every kCacheSteps what is kCacheAge old
 constexpr float kCacheLag = 8.0f;                  // steps a ray may be ahead of the slowest
+// That rule counts steps from the ray's eye and keeps rays of an image side by side.  Rays of a batch
+// without an image width may have their first steps far apart (other cameras, other distances): side by side
+// they would only wait for each other, one after the other.  Up to this spread of first steps such a
+// wavefront keeps the rule, beyond it its rays run freely.  2^18 rays and a 256^3 fog, with the rule, without
+// it, and by spread of 64, 200 and 500 steps: cameras at 16 distances shuffled 7.86, 2.49, 2.49, 2.49, 2.48 ms
+// (accessor 6.38), 128^3: 3.77, 1.18, 1.18, 1.18, 1.86 (3.22); one image as rows of rays 2.82, 3.29, 2.88,
+// 2.79, 2.78 (11.6); 2^20 rays of 16 images in a row 3.25, 4.02, 3.86, 3.41, 3.26 (12.0); scattered rays from one distance
+// 5.01, 5.45, 5.48, 5.47, 5.04 (12.5), from four distances 11.6, 5.40, 5.40, 5.42, 5.42 (12.4).
+constexpr float kCacheSpread = 200.0f;
 constexpr uint32_t kMaxBlockLeaves = 1u << 20;
 
 // float -> int64 fixed point, round to nearest, saturating at +-2^62 (float->int conversion is
@@ -406,7 +415,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     };
     SlotCell c;
     HDDA h;
-    float kf = 0.0f, t = 0.0f, tb = 0.0f;
+    float kf = 0.0f, t = 0.0f, tb = 0.0f, lag = -1.0f; // lag: the wavefront's
     bool pend = false, more = true, first = true;
     if (alive) {
         float p[3];
@@ -440,9 +449,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         if (!__any(pend)) break;
         // rays stay within a few steps of the last one, so that the wavefront's blocks stay few
         const float kmin = waveMinDpp(pend ? kf : kFltMax);
+        if (lag < 0.0f) // every ray with a step at all stands before its first
+            lag = s.width || -waveMinDpp(pend ? -kf : kFltMax) - kmin <= kCacheSpread ? kCacheLag : kFltMax;
 #pragma unroll 1
         for (uint32_t sub = 0; sub < kCacheSteps; ++sub) {
-            const bool act = pend && (kf < kmin + kCacheLag || kf == kmin);
+            const bool act = pend && (kf < kmin + lag || kf == kmin);
             const float x0 = __builtin_fmaf(t, R.dir[0], R.eye[0]), x1 = __builtin_fmaf(t, R.dir[1], R.eye[1]),
                         x2 = __builtin_fmaf(t, R.dir[2], R.eye[2]);
             const float fx = floorf(x0), fy = floorf(x1), fz = floorf(x2);
@@ -558,8 +569,8 @@ int fogMarchBackward(const GridView& g, const float* eye, const float* dir, uint
     TileOrder to;
     SlotMap M;
     // The tiled adjoint wherever the grid has a slot map and its blocks (4 KB per leaf) stay within 4 GiB:
-    // it was the faster one from 1024 rays on, as an image or a scattered batch (1024 rays through a
-    // 256^3 fog: accessor 7.1 ms, blocks 2.9; 1 M scattered rays 23.5 and 10.7).
+    // it was the faster one from 1024 rays on, as an image, a scattered batch or one shuffled over cameras (1024
+    // rays through a 256^3 fog: accessor 7.1 ms, blocks 2.9; 1 M scattered rays from four distances 47.8 and 19.3).
     // Decided before any of it is allocated or built.
     BlockBox X{};
     const bool tiled = g.leafCount && g.leafCount <= kMaxBlockLeaves && sc.tiles < (1u << 26) && blockBoxOf(slotBoxOf(g.bbox), X);

@@ -197,6 +197,29 @@ def _leaf_bytes(host):
     return slice(off, off + 2144 * count)
 
 
+@pytest.mark.parametrize("name", ["fog", "tiles"])
+def test_adjoint_of_rays_far_apart(name):
+    """Wavefronts whose rays' first steps lie farther apart than they march side by side, and nearer: the order
+    of the batch does not change the integers, and an image gives them too."""
+    nvq = _nvq()
+    d = _grid(nvq, _host(nvq, name), "float")
+    lo, hi = np.array(d.index_bbox[:3], np.float64), np.array(d.index_bbox[3:], np.float64) + 1
+    r = np.random.default_rng(6)
+    v = r.normal(size=(4160, 3))
+    far = r.choice([0.0, 0.7, 0.8, 2.0, 12.0], 4160)[:, None]  # times the diagonal: some inside the bbox
+    eye = 0.5 * (lo + hi) + far * np.linalg.norm(hi - lo) * v / np.linalg.norm(v, axis=1, keepdims=True)
+    aim = r.random((4160, 3)) * (hi - lo) + lo + 0.01
+    eye, dirs = (torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).cuda() for x in (eye, aim - eye))
+    gL, gT = (torch.from_numpy(r.normal(size=4160).astype(np.float32)).cuda() for _ in range(2))
+    L, T = nvq.ops.fog_march(d, eye, dirs, 0.5, 0.05)
+    want = nvq.ops.fog_march_backward(d, eye, dirs, L, gL, T, gT, 0.5, 0.05, image_width=65)  # no rule on spread
+    assert int(want.ne(0).sum()) > 1000
+    by_distance = torch.from_numpy(np.argsort(far[:, 0], kind="stable")).cuda()
+    for order in (torch.arange(4160, device="cuda"), by_distance):
+        x = [a[order].contiguous() for a in (eye, dirs, L, gL, T, gT)]
+        assert torch.equal(want, nvq.ops.fog_march_backward(d, *x, 0.5, 0.05))
+
+
 @pytest.mark.parametrize("codec", ["float", "fp8", "fpn"])
 def test_multi_query_over_maps_equals_the_accessor_launch(codec):
     """nvq_multi_query (slot maps, tiles left open answered again) against nvq_multi_query_noalloc."""
