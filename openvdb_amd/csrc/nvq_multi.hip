@@ -200,14 +200,19 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
     const size_t againBytes = 256 + up(size_t(A.totalTiles) * 4), mapBytes = up(sizeof(SlotMap) * kMaxGrids);
     MapJob jobs[kMaxGrids];
     size_t total = need + againBytes + mapBytes, at[kMaxGrids], bytes[kMaxGrids];
+    // maps for all grids where one of them pays on its own: three level sets of 64 rays each 137 us with three
+    // maps, 147 with none, 217 with two
     bool any = false;
     for (uint32_t j = 0; j < A.k; ++j) {
         const MultiSlot& S = A.slot[j];
         jobs[j] = MapJob{views[j], S.view, nullptr, S.op == kOpFogMarch ? kMapBricks : kMapSigns};
-        bytes[j] = S.rayEnd > S.rayBase ? slotMapBytes(*views[j], S.rayEnd - S.rayBase, jobs[j].parts) : 0;
+        any = any || (S.rayEnd > S.rayBase && slotMapBytes(*views[j], S.rayEnd - S.rayBase, jobs[j].parts));
+    }
+    for (uint32_t j = 0; j < A.k; ++j) {
+        const uint64_t rays = A.slot[j].rayEnd - A.slot[j].rayBase;
+        bytes[j] = any && rays ? slotMapBytes(*views[j], rays, jobs[j].parts, true) : 0;
         at[j] = total;
         total += bytes[j];
-        any = any || bytes[j];
     }
     // no map on a captured stream, nor where the scratch cannot grow
     any = any && !isCapturing(s);

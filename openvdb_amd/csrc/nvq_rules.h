@@ -1,6 +1,7 @@
 // Rules on sizes and indices that host code decides by: plain C++, so that tests/test_rules_cpu.py runs them
 // without a GPU.  constexpr functions are callable from kernels too.
 #pragma once
+#include <cmath>
 #include <stdint.h>
 
 namespace nvq {
@@ -47,6 +48,25 @@ inline SlotBox slotBoxOf(const int32_t bbox[6])
     }
     b.count = count;
     return b;
+}
+
+// Whether a crossing's rays pay for a map with sign bits.  A crossing through the accessor takes some hundred
+// microseconds at most, however large its grid, so its map may cost no more than what its walk saves; all in
+// microseconds, fitted to spheres of radius 30, 100, 400 and 800 and a torus (300, 80), 64 to 2^20 rays:
+//   cost: 4 of launches, 45 per million slots, 0.55 per thousand Float leaves read and written (FpN: 1.5, its
+//         leaves being numbered by an atomic)
+//   saved: the grid's extent in slots (cube root of the table) times a factor that grows with the rays: 0.4 at
+//         64 (one 8x8 tile at the torus: 72 us through the accessor, 83 with a map), 1 at 1000, 1.6 at
+//         16,384, 3.1 at 2^18, 5.9 at 2^20
+// Fewer than 64 rays go through the accessor: 17 to 20 us for one, 22 to 31 with a map (FpN torus: 73).
+// 65,536 rays at the sphere of radius 800 (8.5 M slots): 590 us, 609 with a map; 2^18: 760 and 650.
+inline bool crossingMapPays(uint64_t slots, uint64_t leaves, uint32_t leafBytes, bool fpn, uint64_t rays)
+{
+    if (rays < 64) return false;
+    const double perLeaf = fpn ? 1.5e-3 : 0.55e-3 * (leafBytes + 256) / 2400.0;
+    const double cost = 4.0 + 45e-6 * double(slots) + perLeaf * double(leaves);
+    const double saved = std::cbrt(double(slots)) * (0.4 + 0.15 * std::log2(double(rays) / 64.0) + 3.3e-6 * double(rays));
+    return cost <= saved;
 }
 
 // ------------------------------------------------------------------ block cache of the march's adjoint

@@ -160,11 +160,13 @@ __device__ __forceinline__ bool slotTrilinear(const SlotMap& M, float px, float 
     return ok;
 }
 
-// When a map pays: it costs about 45 us per million slots and 1.1 us per 1000 leaves (142 us for the
+// When a map pays.  Marches: it costs about 45 us per million slots and 1.1 us per 1000 leaves (142 us for the
 // 141,950 leaves of a 512^3 fog, 5 TB/s of leaves read and bricks written).  Against that stands the
-// accessor's latency: one ray through that fog takes milliseconds, as its lookups wait for each other.
-// So small launches take a map too, up to these sizes per launch and per ray; beyond them, and
-// where a brick's offset would leave 32 bits, the accessor answers.
+// accessor's latency: one ray through that fog takes 0.4 to 0.7 ms, as its lookups wait for each other, and
+// 0.3 to 0.4 with the map; 64 rays 6.4 and 0.8 ms.  So small launches take a map too, up to these sizes per
+// launch and per ray; beyond them, and where a brick's offset would leave 32 bits, the accessor
+// answers.  (A launch whose rays all miss pays the map for nothing: 15 us and 166.)
+// Crossings: crossingMapPays (nvq_rules.h).
 constexpr uint64_t kMapSlotsPerRay = 256, kMapSlotsFree = 1u << 20;
 constexpr uint64_t kMaxMapLeaves = 1400000, kMapLeavesPerRay = 64, kMapLeavesFree = 1u << 18;
 
@@ -325,8 +327,9 @@ __device__ __forceinline__ bool isoCrossingSlots(const SlotMap& M, const GridVie
 // Host side (nvq_slots.hip).  slotMapBytes: the scratch a map of grid g takes, or 0 when the call
 // should go through the accessor: a bbox or leaf count out of proportion to its rays, or beyond
 // the table's 32-bit offsets.  launchSlotMap builds it in `mem` (256-byte aligned).
-// `parts`: kMapBricks, kMapSigns (against `iso`).
-size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts);
+// `parts`: kMapBricks, kMapSigns (against `iso`).  `besides`: the call builds maps of other grids; a crossing's
+// map then has a march's limits, as its tiles would otherwise wait for the launch after the others'.
+size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts, bool besides = false);
 // One map of a multi-grid call: the grid's view on the host and on the device, and the memory its map
 // is built in (nullptr: none, and maps[j].entry is null).
 struct MapJob {

@@ -275,13 +275,16 @@ bool layMap(const GridView& g, char* mem, uint32_t parts, SlotMap& M, MapMem& W)
 
 } // namespace
 
-size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts)
+size_t slotMapBytes(const GridView& g, uint64_t rays, uint32_t parts, bool besides)
 {
     const uint64_t count = slotBoxOf(g.bbox).count;
     if (!count) return 0;
-    if (count > kMapSlotsPerRay * rays + kMapSlotsFree || g.leafCount > kMapLeavesPerRay * rays + kMapLeavesFree ||
-        g.leafCount > kMaxMapLeaves)
+    if (g.leafCount > kMaxMapLeaves) return 0;
+    if (((parts & kMapBricks) || besides) &&
+        (count > kMapSlotsPerRay * rays + kMapSlotsFree || g.leafCount > kMapLeavesPerRay * rays + kMapLeavesFree))
         return 0;
+    const uint32_t leafBytes = g.type == GT_ONINDEX ? 96u + 2048u : g.leafSize; // with its channel's values
+    if ((parts & kMapSigns) && !besides && !crossingMapPays(count, g.leafCount, leafBytes, g.type == GT_FPN, rays)) return 0;
     const uint64_t leaves = std::max<uint64_t>(g.leafCount, 1);
     return up256(4 * count) * (g.type == GT_ONINDEX ? 3 : 2) + up256(4 * leaves) * 2 + 256 +
            (parts & kMapBricks ? up256(4ull * kBrickFloats * leaves) : 0) + (parts & kMapSigns ? up256(kSignBytes * leaves) : 0);

@@ -91,3 +91,17 @@ def test_adjoint_is_the_same_in_every_form(nvq, name, n):
     for k in ("march only", "none"):
         for a, b in zip(out["map"], out[k]):
             assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("rays,maps", [(63, 0), (64, 1), (4097, 1)])
+def test_crossings_take_a_map_where_it_pays(nvq, rays, maps):
+    """Around the number of rays from which a sphere's crossing takes a map; the smaller call is the larger one's
+    first rays, through the accessor."""
+    d = nvq.DeviceGrid(nvq.tools.create_level_set_sphere(37.0, (1.5, -2.0, 3.0), 1.0, 3.0))
+    eye, dirs = _rays(rays, 5)
+    got, built = _launches(nvq, "slot_map", lambda: nvq.ops.zero_crossing(d, eye, dirs))
+    assert built == maps
+    part, built = _launches(nvq, "slot_map", lambda: nvq.ops.zero_crossing(d, eye[:63].contiguous(), dirs[:63].contiguous()))
+    assert built == 0
+    for a, b in zip(got, part):
+        assert torch.equal(a[:63].contiguous().view(torch.uint8), b.view(torch.uint8))

@@ -106,3 +106,22 @@ def test_fd6_samples_below_2_23_stay_near_their_block():
     assert off.sum() > 100
     first, last, far = (cell - 1) >> 3, (cell + 2) >> 3, (cell + up + 1) >> 3
     assert np.all((far == first) | (far == last))
+
+
+# (slots, leaves, bytes per leaf, FpN), rays, whether the crossing was measured faster with the map
+LEVEL_SETS = {"sphere30": (1728, 345, 2144, 0), "sphere100": (24389, 4025, 2144, 0), "torus300": (235224, 30249, 2144, 0),
+              "torus300fp16": (235224, 30249, 1120, 0), "torus300fpn": (235224, 30249, 0, 1),
+              "sphere400": (1124864, 64800, 2144, 0), "sphere800": (8489664, 259616, 2144, 0)}
+
+
+@pytest.mark.parametrize("name,rays,pays", [
+    ("sphere30", 1, 0), ("sphere30", 8, 0), ("sphere30", 64, 1), ("sphere30", 1000, 1), ("sphere30", 1 << 20, 1),
+    ("sphere100", 4, 0), ("sphere100", 16, 0), ("sphere100", 64, 1), ("sphere100", 16384, 1),
+    ("torus300", 1, 0), ("torus300", 16, 0), ("torus300", 64, 0), ("torus300", 256, 1), ("torus300", 1 << 18, 1),
+    ("torus300fp16", 1000, 1), ("torus300fpn", 64, 0), ("torus300fpn", 128, 0), ("torus300fpn", 1 << 20, 1),
+    ("sphere400", 64, 0), ("sphere400", 1000, 1), ("sphere400", 1 << 18, 1),
+    ("sphere800", 16384, 0), ("sphere800", 65536, 0), ("sphere800", 1 << 18, 1), ("sphere800", 1 << 20, 1)])
+def test_crossing_maps_are_built_where_they_were_faster(tmp_path, name, rays, pays):
+    slots, leaves, size, fpn = LEVEL_SETS[name]
+    out = run_cpp(tmp_path, f'std::printf("%d\\n", crossingMapPays({slots}u, {leaves}u, {size}u, {"true" if fpn else "false"}, {rays}u));')
+    assert int(out[0]) == pays
