@@ -376,12 +376,12 @@ int makeMultiArgs(const nvq_grid* const* host_grids, uint32_t k, const uint64_t*
 // wavefronts in flight share one region of the grids) while the atomics are spread over 8
 // addresses instead of serialising on one.  A wavefront starts on its XCD's counter and moves to
 // the next once that counter's chunks pass the end; it returns after all 8, so every wavefront
-// exits.  Without counters (a captured launch that gets no scratch) the wavefronts take the tiles in
-// turn.
+// exits.  kMayLack: without counters (a captured launch that gets no scratch) the wavefronts take the
+// tiles in turn; only compiled where that can be (in every loop it cost 1.5 %).
 constexpr uint32_t kQueueBands = 8, kQueueStride = 64, kQueueChunk = 1; // stride in uint32 (256 B)
 constexpr size_t kQueueBytes = size_t(kQueueBands) * kQueueStride * sizeof(uint32_t);
 
-template<class F>
+template<bool kMayLack = false, class F>
 __device__ __forceinline__ void forEachQueuedTile(uint32_t* __restrict__ counters, uint32_t total, F&& f)
 {
     const uint32_t lane = threadIdx.x & 63u, home = blockIdx.x & (kQueueBands - 1);
@@ -390,7 +390,7 @@ __device__ __forceinline__ void forEachQueuedTile(uint32_t* __restrict__ counter
         const uint32_t r = (home + k) & (kQueueBands - 1);
         for (uint32_t i = 0;; ++i) {
             uint64_t q;
-            if (counters) {
+            if (!kMayLack || counters) {
                 uint32_t b = 0;
                 if (lane == 0) b = atomicAdd(counters + r * kQueueStride, 1u);
                 b = __shfl(b, 0, 64);
@@ -402,7 +402,7 @@ __device__ __forceinline__ void forEachQueuedTile(uint32_t* __restrict__ counter
             const uint32_t t0 = uint32_t(q) * kQueueChunk, t1 = t0 + kQueueChunk < total ? t0 + kQueueChunk : total;
             for (uint32_t t = t0; t < t1; ++t) f(t);
         }
-        if (!counters) break;
+        if (kMayLack && !counters) break;
     }
 }
 

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kBlock) void k_multi_query(MultiArgs A, const float
                                                         uint32_t* __restrict__ counters,
                                                         const uint32_t* __restrict__ order, CrossingOut o)
 {
-    forEachQueuedTile(counters, A.totalTiles, [&](uint32_t q) { runTile(A, order ? order[q] : q, eye, dir, dt, sigma, o); });
+    forEachQueuedTile<true>(counters, A.totalTiles, [&](uint32_t q) { runTile(A, order ? order[q] : q, eye, dir, dt, sigma, o); });
 }
 
 // The same over slot maps: one march and one crossing body for every codec.  A tile with a ray its map
