@@ -571,9 +571,12 @@ int fogMarchBackward(const GridView& g, const float* eye, const float* dir, uint
     // The tiled adjoint wherever the grid has a slot map and its blocks (4 KB per leaf) stay within 4 GiB:
     // it was the faster one from 1024 rays on, as an image, a scattered batch or one shuffled over cameras (1024
     // rays through a 256^3 fog: accessor 7.1 ms, blocks 2.9; 1 M scattered rays from four distances 47.8 and 19.3).
+    // Not for fewer than four rays, whose march does not make up for the map, the clearing and the folding of
+    // 4 KB per leaf: 1, 2, 4 and 8 rays through a 512^3 fog 0.70, 1.38, 2.45 and 3.86 ms through the
+    // accessor, 1.17, 1.56, 2.05 and 2.42 with blocks.
     // Decided before any of it is allocated or built.
     BlockBox X{};
-    const bool tiled = g.leafCount && g.leafCount <= kMaxBlockLeaves && sc.tiles < (1u << 26) && blockBoxOf(slotBoxOf(g.bbox), X);
+    const bool tiled = n >= 4 && g.leafCount && g.leafCount <= kMaxBlockLeaves && sc.tiles < (1u << 26) && blockBoxOf(slotBoxOf(g.bbox), X);
     const uint64_t blockBytes = tiled ? uint64_t(g.leafCount) * 4096u : 0;
     if (tileOrder(g, eye, dir, sc, to, s, 256, tiled ? &M : nullptr, blockBytes) != 0) return -1;
     uint32_t* flag = reinterpret_cast<uint32_t*>(to.extra);

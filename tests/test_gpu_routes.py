@@ -93,6 +93,22 @@ def test_adjoint_is_the_same_in_every_form(nvq, name, n):
             assert torch.equal(a, b), k
 
 
+def test_adjoint_of_few_rays(nvq):
+    """Three rays through the accessor, four with the block cache: the fourth's gradients are zero."""
+    d = nvq.DeviceGrid(_host(nvq, "fog"))
+    eye, dirs = _rays(8, 2)  # the first inside the fog
+    eye, dirs = eye[:4].contiguous(), dirs[:4].contiguous()
+    gL = torch.tensor([1.0, -2.0, 0.5, 0.0], device="cuda")
+    L, T = nvq.ops.fog_march(d, eye, dirs, 0.5, 0.05)
+    out = []
+    for n, maps in ((4, 1), (3, 0)):
+        x = [a[:n].contiguous() for a in (eye, dirs, L, gL, T, gL)]
+        acc, built = _launches(nvq, "slot_map", lambda: nvq.ops.fog_march_backward(d, *x, 0.5, 0.05))
+        assert built == maps
+        out.append(acc)
+    assert torch.equal(*out) and int(out[0].ne(0).sum()) > 10
+
+
 @pytest.mark.parametrize("rays,maps", [(63, 0), (64, 1), (4097, 1)])
 def test_crossings_take_a_map_where_it_pays(nvq, rays, maps):
     """Around the number of rays from which a sphere's crossing takes a map; the smaller call is the larger one's
