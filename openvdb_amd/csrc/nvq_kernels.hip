@@ -107,7 +107,13 @@ __global__ __launch_bounds__(kBlock) void k_get_value(GridView g, const int32_t*
 // The same over a slot table: two lookups (slot, leaf) instead of the walk's five.  Voxels outside the
 // table, or in a slot it leaves open, go through the tree.  Bound by the L1's and L2's line rate: 10.6 M
 // shuffled voxels of an index grid 443 -> 370 us (two or four voxels per lane at a time: the same).
-constexpr uint64_t kValueMapMin = 1u << 18;
+// From 2^22 voxels on, where the table's 3 to 25 us are made up for: walk and table take 77 and 76 us for 2^22
+// random voxels of a 256^3 fog, 40 and 35 of a 64^3, 131 and 121 of a 512^3, 27 and 25 for the active
+// voxels of a torus in order; 2^20 voxels 23 and 26.  (Batches mostly outside the grid, whose walk ends at
+// the root, lose those microseconds.)  Up to 2^19 slots, 4 MB of entries and values, an XCD's L2: 2^24
+// random voxels through 1.1 M slots took 411 us instead of 355.  Not for FpN, whose leaves the table
+// numbers one by one: 85 and 99 us for 2^22 voxels of the 256^3 fog, 362 and 387 for 2^24.
+constexpr uint64_t kValueMapMin = 1u << 22, kValueMapSlots = 1u << 19;
 template<uint32_t GT>
 __global__ __launch_bounds__(kBlock) void k_get_value_slots(SlotMap M, GridView g, const int32_t* __restrict__ ijk,
                                                             uint64_t n, float* __restrict__ val,
@@ -336,10 +342,14 @@ template<uint32_t GT> struct RunGetValue {
     static void run(const GridView& g, const SlotMap* M, const int32_t* ijk, uint64_t n, float* val, uint8_t* act,
                     uint32_t* dim, hipStream_t s)
     {
-        if (M)
-            hipLaunchKernelGGL(k_get_value_slots<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, *M, g, ijk, n, val, act, dim);
-        else
-            hipLaunchKernelGGL(k_get_value<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, g, ijk, n, val, act, dim);
+        if constexpr (GT != GT_FPN) {
+            if (M) {
+                hipLaunchKernelGGL(k_get_value_slots<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, *M, g, ijk, n, val,
+                                   act, dim);
+                return;
+            }
+        }
+        hipLaunchKernelGGL(k_get_value<GT>, dim3(gridStrideBlocks(n)), dim3(kBlock), 0, s, g, ijk, n, val, act, dim);
     }
 };
 template<uint32_t GT> struct RunSample {
@@ -825,13 +835,13 @@ int nvq_get_value(const nvq_grid* grid, const int32_t* ijk, uint64_t n, float* v
 {
     if (!grid || !queryable(grid) || (n && !ijk)) return NVQ_ERR_INVALID_ARG;
     if (n == 0) return NVQ_OK;
-    // Large batches through a slot table: about 45 us per million slots to build, against about 7 us saved per
-    // million voxels, so from 8 voxels per slot on.
+    // large batches through a slot table (k_get_value_slots)
     WorkspaceLease lease;
     SlotMap M;
     bool mapped = false;
-    const uint64_t slots = n >= kValueMapMin ? slotBoxOf(grid->view.bbox).count : 0;
-    if (slots && slots <= n / 8)
+    const bool large = n >= kValueMapMin && grid->view.type != GT_FPN;
+    const uint64_t slots = large ? slotBoxOf(grid->view.bbox).count : 0;
+    if (slots && slots <= kValueMapSlots)
         (void)acquireWithMap(lease, grid->view, n, 0u, 0.0f, 0, 0, M, mapped, S(stream));
     return launchTyped<RunGetValue>(grid->view.type, grid->view, mapped ? &M : nullptr, ijk, n, val, active, dim, S(stream));
 }

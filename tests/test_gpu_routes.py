@@ -8,7 +8,7 @@ import ctypes
 
 import numpy as np
 import pytest
-from test_gpu_slots import _host
+from test_gpu_slots import _grid, _host, _level_set
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -121,3 +121,51 @@ def test_crossings_take_a_map_where_it_pays(nvq, rays, maps):
     assert built == 0
     for a, b in zip(got, part):
         assert torch.equal(a[:63].contiguous().view(torch.uint8), b.view(torch.uint8))
+
+
+def _voxels(d, n, seed):
+    """Inside leaves, on tiles and background in the bbox, on the table's rim, around it, far out, at the ends of
+    the integer range; n not a multiple of a wavefront."""
+    r = np.random.default_rng(seed)
+    lo, hi = np.array(d.index_bbox[:3], np.int64), np.array(d.index_bbox[3:], np.int64) + 1
+    ijk = r.integers(lo - 3, hi + 3, (n, 3))
+    k = n // 16
+    ijk[:k] = r.integers(lo - 40, hi + 40, (k, 3))
+    ijk[k:2 * k] = r.integers(-2 ** 31, 2 ** 31, (k, 3))
+    rim = np.stack([(lo >> 3 << 3) - 9, (lo >> 3 << 3) - 8, (hi >> 3 << 3) + 15, (hi >> 3 << 3) + 16, (hi >> 3 << 3) + 24])
+    ijk[2 * k:3 * k] = np.where(r.random((k, 3)) < 0.5, rim[r.integers(0, 5, k)], ijk[2 * k:3 * k])
+    ends = np.array([-2 ** 31, -2 ** 31 + 7, 2 ** 31 - 1, 2 ** 31 - 8, -1, 0])
+    ijk[3 * k:3 * k + 512] = r.choice(ends, (512, 3))
+    return np.ascontiguousarray(ijk.astype(np.int32))
+
+
+@pytest.mark.parametrize("name,codec", [("fog", c) for c in ("float", "fp4", "fp8", "fp16", "fpn", "onindex")] +
+                         [("tiles", "float"), ("tiles", "fp8"), ("flagged", "float"), ("sphere", "fp16")])
+def test_large_value_batches_equal_small_ones(nvq, oracle, name, codec):
+    """getValue through the slot table (from 2^22 voxels on, not FpN) against the same voxels in smaller batches
+    through the tree, and against the oracle."""
+    host = _level_set(nvq, name) if name == "sphere" else _host(nvq, name)
+    d = _grid(nvq, host, codec)
+    n = (1 << 22) + 37
+    ijk = _voxels(d, n, 3)
+    x = torch.from_numpy(ijk).cuda()
+    got, maps = _launches(nvq, "slot_map", lambda: nvq.ops.get_value(d, x, want_dim=True))
+    assert maps == (0 if codec == "fpn" else 1)
+    pieces, maps = _launches(nvq, "slot_map", lambda: [nvq.ops.get_value(d, y.contiguous(), want_dim=True) for y in x.split(1 << 21)])
+    assert maps == 0
+    for a, b in zip(got, zip(*pieces)):
+        assert torch.equal(a.view(torch.uint8), torch.cat(b).view(torch.uint8))
+    if codec == "float":
+        for a, b in zip(got, oracle.get_value(host, ijk[:300000])):
+            assert np.array_equal(a[:300000].cpu().numpy().view(np.uint8), np.ascontiguousarray(b).view(np.uint8))
+    assert 1000 < int(got[1].sum()) < n
+
+
+def test_value_table_limits(nvq):
+    """One voxel below the batch size, and a box of more slots than the table takes: through the tree."""
+    d = nvq.DeviceGrid(_host(nvq, "fog"))
+    x = torch.zeros(1 << 22, 3, dtype=torch.int32, device="cuda")
+    assert _launches(nvq, "slot_map", lambda: nvq.ops.get_value(d, x[:-1]))[1] == 0
+    assert _launches(nvq, "slot_map", lambda: nvq.ops.get_value(d, x))[1] == 1
+    wide = nvq.DeviceGrid(nvq.aligned_buffer(_stretched(_host(nvq, "fog"), 8 * 78)))  # 81^3 slots
+    assert _launches(nvq, "slot_map", lambda: nvq.ops.get_value(wide, x))[1] == 0
