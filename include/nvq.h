@@ -5,13 +5,17 @@
  * "host_", every pointer argument is a DEVICE pointer.  A `stream` is a
  * hipStream_t passed as void* (NULL = the default stream).  Every call is
  * stream-ordered and asynchronous unless its comment says it waits.  Every call returns NVQ_OK (0)
- * or a negative NVQ_ERR_* status.  Nothing throws across the ABI.  Query scratch (ray-tile orders,
- * queue counters, slot maps of ray queries: about 3 KB per leaf, the sort buffers of binned point
- * queries) lives in one grow-only block per (device, stream) that the library keeps until the
- * process ends; ray queries take no slot map on a stream under graph capture, or where the block
- * cannot grow, and give the same bits without it.  A captured call uses its stream's block as it is, or
- * runs without scratch where that is too small, and the block it uses is kept for the graph's replays;
- * replay such a graph on the stream it was captured on, or not beside other calls on that stream.
+ * or a negative NVQ_ERR_* status.  Nothing throws across the ABI.  Query scratch lives in one
+ * grow-only block per (device, stream) that the library keeps until the process ends, sized for the
+ * largest call on that stream plus an eighth (at most 256 MiB): ray-tile orders and queue counters,
+ * the sort buffers of binned point queries (about 110 bytes per point), and the slot maps of ray
+ * queries and large getValue batches.  A map takes 8 bytes per 8^3 slot of the grid's bbox (12 on
+ * index grids) and per leaf about 3 KB for a march, 7 KB for its adjoint and 300 bytes for
+ * crossings; one call's maps take at most 8 GiB.  No map is taken on a stream under graph capture,
+ * beyond that, or where the block cannot grow; the results are the same bits without it.  A captured
+ * call uses its stream's block as it is, or runs without scratch where that is too small, and the
+ * block it uses is kept for the graph's replays; replay such a graph on the stream it was captured
+ * on, or not beside other calls on that stream.
  * Besides the block, the library holds
  * the opt-in kernel profiler (nvq_profile_*), the work-queue array of nvq_multi_query_noalloc and
  * a small pinned host buffer per calling thread for values it reads back.  Calls on distinct

@@ -638,7 +638,7 @@ char* nvq::acquireWithMap(WorkspaceLease& lease, const GridView& g, uint64_t ray
     const size_t at = ((need + 255) & ~size_t(255)) + ((withMap + 255) & ~size_t(255));
     const size_t mapBytes = slotMapBytes(g, rays, parts);
     // a captured launch takes the accessor, whatever scratch the stream happens to hold
-    if (mapBytes && !isCapturing(st)) {
+    if (mapBytes && mapBytes + withMap <= kMaxMapBytes && !isCapturing(st)) {
         char* base = lease.acquire(at + mapBytes, st, true);
         if (base) {
             mapped = launchSlotMap(g, base + at, M, parts, iso, st) == 0;

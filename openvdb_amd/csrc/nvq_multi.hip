@@ -211,6 +211,9 @@ int multiQuery(const MultiArgs& A, const GridView* const* views, const float* ey
     for (uint32_t j = 0; j < A.k; ++j) {
         const uint64_t rays = A.slot[j].rayEnd - A.slot[j].rayBase;
         bytes[j] = any && rays ? slotMapBytes(*views[j], rays, jobs[j].parts, true) : 0;
+    }
+    boundMaps(bytes, A.k);
+    for (uint32_t j = 0; j < A.k; ++j) {
         at[j] = total;
         total += bytes[j];
     }

@@ -2,6 +2,7 @@
 // without a GPU.  constexpr functions are callable from kernels too.
 #pragma once
 #include <cmath>
+#include <stddef.h>
 #include <stdint.h>
 
 namespace nvq {
@@ -48,6 +49,19 @@ inline SlotBox slotBoxOf(const int32_t bbox[6])
     }
     b.count = count;
     return b;
+}
+
+// The scratch that one call may take for maps and what goes with them (the adjoint's blocks): a stream keeps
+// its block until the process ends.  A march's map is 2.9 KB per leaf, the adjoint's and its blocks 7 KB:
+// 1.4 M and 2^20 leaves, the most they are built for, stay within it; of a multi-grid call's maps those that
+// still fit are built, in order, and the other grids' tiles go through the accessor.
+constexpr uint64_t kMaxMapBytes = uint64_t(8) << 30;
+inline void boundMaps(size_t* bytes, uint32_t n, uint64_t most = kMaxMapBytes)
+{
+    for (uint32_t j = 0; j < n; ++j) {
+        if (bytes[j] > most) bytes[j] = 0;
+        most -= bytes[j];
+    }
 }
 
 // Whether a crossing's rays pay for a map with sign bits.  A crossing through the accessor takes some hundred

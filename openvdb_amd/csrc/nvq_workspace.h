@@ -31,7 +31,9 @@ char* scratchAcquire(ScratchBlock& b, size_t bytes, bool capturing, bool optiona
     if (!b.ptr || b.bytes < bytes) {
         if (capturing) return nullptr;
         if (optional && b.refused && bytes >= b.refused && ++b.asked % kRefusedAgain) return nullptr;
-        const size_t grown = bytes + bytes / 8, least = size_t(1) << 20, want = grown > least ? grown : least;
+        // room to grow: an eighth, at most 256 MiB
+        const size_t eighth = bytes / 8, most = size_t(256) << 20, least = size_t(1) << 20;
+        const size_t grown = bytes + (eighth < most ? eighth : most), want = grown > least ? grown : least;
         auto drop = [&]() {
             if (b.ptr && !b.captured) mem.free(b.ptr);
             b.ptr = nullptr;

@@ -125,3 +125,18 @@ def test_crossing_maps_are_built_where_they_were_faster(tmp_path, name, rays, pa
     slots, leaves, size, fpn = LEVEL_SETS[name]
     out = run_cpp(tmp_path, f'std::printf("%d\\n", crossingMapPays({slots}u, {leaves}u, {size}u, {"true" if fpn else "false"}, {rays}u));')
     assert int(out[0]) == pays
+
+
+@pytest.mark.parametrize("wanted,built", [([3, 4, 1], [3, 4, 1]), ([9], [0]), ([8], [8]), ([5, 4, 3, 1], [5, 0, 3, 0]),
+                                          ([0, 0, 8, 1], [0, 0, 8, 0])])
+def test_maps_of_a_call_are_bounded(tmp_path, wanted, built):
+    """In GiB, against the 8 that one call may take."""
+    sizes = ", ".join(f"size_t({w}) << 30" for w in wanted)
+    out = run_cpp(tmp_path, f"""
+    size_t b[] = {{{sizes}}};
+    boundMaps(b, {len(wanted)}u);
+    for (size_t x : b) std::printf("%zu\\n", x >> 30);
+    // the largest map of a march and of an adjoint fit, with a slot table of 2^24
+    std::printf("%d\\n", 1400000ull * (2944 + 8) + (12ull << 24) + 4096 <= kMaxMapBytes &&
+                         (1ull << 20) * (2944 + 8 + 4096) + (12ull << 23) + 4096 <= kMaxMapBytes ? 1 : 0);""")
+    assert [int(x) for x in out] == built + [1]

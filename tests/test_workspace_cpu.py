@@ -28,6 +28,7 @@ def test_block_is_reused_and_grows(tmp_path):
     char* q = scratchAcquire(b, 16 * MB, false, false, m);
     say(q && q != p && b.bytes == 18 * MB && m.frees == 1 && m.freed[0] == p);
     say(scratchAcquire(b, 5, false, false, m) == q && m.allocs == 2);
+    say(scratchAcquire(b, 8192 * MB, false, false, m) && b.bytes == 8448 * MB); // an eighth, at most 256 MiB
     """)
 
 
