@@ -5,7 +5,7 @@ A launch under graph capture takes no scratch and goes through the accessor, so 
 the reference here; the march itself is compared with the FP64 oracle in test_gpu_parity.py.
 Covered: every codec, active tiles, leaves and nodes under render-skip flags (which the map leaves to
 the accessor), bboxes that start and end inside a leaf, steps that round off their slot, rays that
-start inside, run along an axis or miss, and launches of one ray up to several tiles.
+start inside, run along an axis or miss, and launches of one ray up to more tiles than take four lanes per ray.
 """
 import gc
 
@@ -80,15 +80,10 @@ def _rays(d, n):
 def test_march_over_slots_equals_march_through_the_accessor(name, codec):
     nvq = _nvq()
     d = _grid(nvq, _host(nvq, name), codec)
-    for n, dt in ((1, 0.5), (65, 0.37), (4097, 0.5), (4096, 1.9), (1 << 19, 0.5), ((1 << 19) + 65, 0.37)):
+    for n, dt in ((1, 0.5), (65, 0.37), (4097, 0.5), (4096, 1.9)):
         eye, dirs = _rays(d, n)
         L, T = nvq.ops.fog_march(d, eye, dirs, dt, 0.05)
         torch.cuda.synchronize()
-        if n > 1 << 18:  # around the launch size from which a ray takes one lane: larger than a capture
-            if codec == "float":  # without scratch takes, so against its first rays
-                a, b = nvq.ops.fog_march(d, eye[:4099].contiguous(), dirs[:4099].contiguous(), dt, 0.05)
-                assert torch.equal(L[:4099], a) and torch.equal(T[:4099], b)
-            continue
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph):
             Lc, Tc = nvq.ops.fog_march(d, eye, dirs, dt, 0.05)
@@ -103,6 +98,37 @@ def test_march_over_slots_equals_march_through_the_accessor(name, codec):
             assert torch.equal(L, L2)
         if n > 64:
             assert float(L.max()) > 0.0
+
+
+QUAD_RAYS = 64 * 8192  # the march takes four lanes per ray up to here, one lane from there on
+
+
+@pytest.mark.parametrize("name,codec", [("fog", c) for c in ("float", "fp4", "fp8", "fp16", "fpn", "onindex")] +
+                         [("tiles", "float"), ("flagged", "float")])
+def test_one_lane_march_equals_four(name, codec):
+    """Launches above that size, whole, against the same rays in launches below it (which the test above compares
+    with the accessor): a linear batch with a ragged last tile and an image."""
+    nvq = _nvq()
+    d = _grid(nvq, _host(nvq, name), codec)
+    n = QUAD_RAYS + 65
+    eye, dirs = _rays(d, n)
+    L, T = nvq.ops.fog_march(d, eye, dirs, 0.37, 0.05)
+    parts = [nvq.ops.fog_march(d, e.contiguous(), x.contiguous(), 0.37, 0.05)
+             for e, x in zip(eye.split(QUAD_RAYS // 2 + 7), dirs.split(QUAD_RAYS // 2 + 7))]
+    for a, b in zip((L, T), zip(*parts)):
+        assert torch.equal(a.view(torch.int32), torch.cat(b).view(torch.int32))
+    assert int((L > 0.0).sum()) > n // 8
+    first = nvq.ops.fog_march(d, eye[:4099].contiguous(), dirs[:4099].contiguous(), 0.37, 0.05)  # in image order
+    assert torch.equal(L[:4099], first[0]) and torch.equal(T[:4099], first[1])
+    w, h = 1021, 517  # 128 x 65 tiles
+    eye, dirs = _image(d, w, h)
+    L, T = nvq.ops.fog_march(d, eye, dirs, 0.5, 0.05, image_width=w)
+    rows = 200 * w
+    parts = [nvq.ops.fog_march(d, e.contiguous(), x.contiguous(), 0.5, 0.05, image_width=w)
+             for e, x in zip(eye.split(rows), dirs.split(rows))]
+    for a, b in zip((L, T), zip(*parts)):
+        assert torch.equal(a.view(torch.int32), torch.cat(b).view(torch.int32))
+    assert int((L > 0.0).sum()) > 1000
 
 
 def _level_set(nvq, name):
