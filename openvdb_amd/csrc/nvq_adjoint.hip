@@ -234,8 +234,8 @@ __device__ __forceinline__ void blockAdd(const SlotMap& M, const GridView& g, un
 // than kCacheLag steps ahead of the slowest), every step one flush of the whole wavefront.  The
 // accumulator's own order splits a block over four 64-byte lines, so the blocks go to scratch and
 // k_fold_blocks adds them up afterwards; integer sums, so the order does not matter.
-// 10.6 ms for the 64 x 256^2 rays (36.2 ms through the accessor), bound by the VALU (5.6 G wavefront
-// instructions, about 450 per step) at 4 wavefronts per SIMD.
+// 10.6 ms for the 64 x 256^2 rays (36.2 ms through the accessor), bound by the VALU at 4 wavefronts per SIMD:
+// 4.85 G wavefront instructions, 81 % of the issue slots of busy CUs.
 template<uint32_t GT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_fog_march_bwd_blocks(SlotMap M, BlockBox X, GridView g, const float* __restrict__ eye,
                                                              const float* __restrict__ dir, Sched s,

@@ -17,7 +17,8 @@
 //                    LDS, a row of eight voxels per load (ReadAccessor::getValue semantics, so results are bit-identical) and
 //                    evaluates the bin's queries from it; each query's results go to its original
 //                    index as one 64-byte record, written by the four lanes of a quad
-//   k_sample_list  : queries whose stencil leaves the brick run through the lane accessor
+//   k_sample_list  : queries whose stencil leaves the brick, or whose FD6 samples can lie two cells away
+//                    (coordinates from 2^23 on), one per lane over the tree
 //   k_bin_finish   : the outputs in caller order: marked queries copy their record, the others
 //                    (their block has no leaf) are evaluated from the slot table's values
 // On MI355X a random store is cheap only when one instruction writes a whole aligned 64-byte block
@@ -903,9 +904,9 @@ void launchClassify(const GridView& g, const Bins& B, const SlotTable& T, float*
     ProfScope prof("k_bin_classify", s);
     const uint64_t words = (count + 31) / 32;
     const uint32_t ldsWords = words <= kLdsLeafWords ? uint32_t(words) : 0u;
-    // A large bitmap is staged by no more workgroups than the CUs' LDS holds at once: the 41 KB of a 512^3
-    // fog took 198 us with 4096 workgroups (168 MB staged in all) and 160 us with 768; the 26 KB of
-    // the torus 343 us with 4096 and 355 with 1536, so smaller ones keep the workgroups
+    // A large bitmap is staged by no more workgroups than the CUs' LDS holds at once.  Calls of 2^24 points with
+    // 4096 workgroups and with that many: bitmap of 46 KB 718 and 674 us, 38 KB 724 and 692, 32 KB 693 and 683,
+    // 26 KB 650 and 644, 21 KB 643 and 649, 19 KB 649 and 655; 2^20 points the same within 1 % throughout
     if (ldsWords > 8192u) blocks = std::min<uint32_t>(blocks, 256u * ((160u << 10) / (ldsWords * 4u + 64u)));
     hipLaunchKernelGGL(k_bin_classify, dim3(blocks), dim3(kThreads), size_t(ldsWords) * 4u, s, g, T, xyz, B.n, B.chunks,
                        world, c.mode, ldsWords, B.cflags, B.counts);

@@ -146,8 +146,9 @@ __global__ __launch_bounds__(kBlock) void k_get_value_slots(SlotMap M, GridView 
 }
 
 // ------------------------------------------------------------------ point sampling
-// 4 wavefronts per SIMD (128 VGPRs, a spill of 56 to 116 bytes): 300,007 queries take 54.6 us, 1000 take 11.7.
-// Uncapped (171 VGPRs, 2 wavefronts) an earlier form took 64.2 instead of 58.8, and 12.1 instead of 12.4.
+// 4 wavefronts per SIMD (128 VGPRs, a spill of 56 to 116 bytes): 1000 and 300,007 points around a torus, FD6,
+// 12.9 and 82.4 us, 13.1 and 83.0 uncapped (2 wavefronts); 12.6 and 34.8 with the trilinear gradient, 13.1
+// and 36.1 uncapped.  Half of them spread over the bbox: 11.7 and 54.7.
 // Bound by the L1's line rate for the larger, by the chain of five lookups for the smaller.
 template<uint32_t GT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_sample(GridView g, const float* __restrict__ xyz, uint64_t n, int world,

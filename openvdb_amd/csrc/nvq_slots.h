@@ -8,8 +8,8 @@
 //   entry[slot] : for every 8^3 slot of the grid's bbox (one slot wider below, two above) the leaf
 //                 that holds it, or the getDim and state of the tile that covers it
 //   value[slot] : the value every voxel of a slot without a leaf reads (tile or background)
-//   brick[leaf] (marches) : 9^3 decoded floats, the leaf's voxels and the next one of its upper neighbours, so
-//                 that the eight corners of any cell that starts in the leaf are four 8-byte loads
+//   brick[leaf] (marches) : 9^3 decoded floats, the leaf's voxels and the next one of its upper
+//                 neighbours, so that the eight corners of any cell that starts in the leaf are four 8-byte loads
 //                 from one base address, whatever the codec
 //   signs[leaf] (crossings) : per 4^3 block of the leaf the active bits of its voxels and the bits
 //                 of those below and above the iso value, so that a ray walking through the narrow
