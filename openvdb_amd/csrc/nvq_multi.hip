@@ -73,7 +73,8 @@ __global__ __launch_bounds__(kBlock) void k_multi_query(MultiArgs A, const float
 // gain more from wavefronts than the marches from batches.  Sixteen Fp16 grids, 16.8 M rays: accessor
 // 5.65 ms; 4 steps and 3 wavefronts 2.83, 4 and 4 2.51, 2 and 4 2.31, 2 and 6 2.24, 1 and 7 2.17.
 // Marches alone, three fogs of 64^2, 256^2 and 1024^2 rays each: 0.86, 0.69 and 1.24 ms (accessor 3.8, 2.9, 5.3).
-// Sixteen Fp16 grids: the VALU issues in 86 % of the slots of busy CUs, 21 % of wavefront cycles wait.
+// Sixteen Fp16 grids: the VALU issues in 86 % of the slots of busy CUs, 21 % of wavefront
+// cycles wait to issue.
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(7, 8))) void k_multi_slots(MultiArgs A, const SlotMap* __restrict__ maps,
                                                         const float* __restrict__ eye, const float* __restrict__ dir,
                                                         float dt, float sigma, uint32_t* __restrict__ counters,

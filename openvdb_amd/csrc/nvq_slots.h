@@ -162,8 +162,8 @@ __device__ __forceinline__ bool slotTrilinear(const SlotMap& M, float px, float 
 
 // When a map pays.  Marches: it costs about 45 us per million slots and 1.1 us per 1000 leaves (142 us for the
 // 141,950 leaves of a 512^3 fog, 5 TB/s of leaves read and bricks written).  Against that stands the
-// accessor's latency: one ray through that fog takes 0.4 to 0.7 ms, as its lookups wait for each other, and
-// 0.3 to 0.4 with the map; 64 rays 6.4 and 0.8 ms.  So small launches take a map too, up to these sizes per
+// accessor's latency: one ray through that fog takes 0.39 to 0.49 ms, as its lookups wait for each other,
+// and 0.30 to 0.36 with the map; 64 rays 6.4 and 0.8 ms.  So small launches take a map too, up to these sizes per
 // launch and per ray; beyond them, and where a brick's offset would leave 32 bits, the accessor
 // answers.  (A launch whose rays all miss pays the map for nothing: 15 us and 166.)
 // Crossings: crossingMapPays (nvq_rules.h).
